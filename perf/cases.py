@@ -146,7 +146,7 @@ def tolerance(case):
     n = 24, 1.9e-6 at 100, 1.3e-5 at 430, 2.0e-5 at 512. The 64-bit types' are these times
     the ratio of the roundings (gradients 1.8e-15 at n = 63)."""
     unit = 1.0 if case["dtype"] in ("f32", "c64") else 2.0**-29
-    rel = 1.5e-6
+    rel = 4.0e-6 if case["dtype"].startswith("c") else 1.5e-6
     if case["grad"]:
         rel = 5.0e-6 if case["op"] in ("slogpf", "pf") else max(5.0e-6, 1.6e-7 * case["n"])
     return {"rel": rel * unit, "max": 100 * rel * unit}
