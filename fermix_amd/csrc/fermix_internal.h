@@ -110,6 +110,17 @@ int launch_lu_inverse(float* LU, const int* g0, int N, int n, int64_t batch, con
                       int zero_singular, float* invT, bool in_place, void* ws, size_t ws_bytes,
                       hipStream_t s, const float* scale = nullptr, int x3 = 0);
 
+// The same from padded orders N <= SMALL_INV_MAXN (a multiple of 16) in one launch each, read
+// only, no workspace (small_inverse.hip): launch_lu_inverse's A^-T or, with det, adj(A)^T =
+// d det / dA (sign / logabs the factorisation's own; scale unused), and launch_pf_inverse's
+// results.
+constexpr int SMALL_INV_MAXN = 128;
+int launch_lu_inv_small(const float* LU, const int* g0, int N, int n, int64_t batch, const float* sign,
+                        const float* logabs, const float* scale, int zero_singular, bool det, float* out,
+                        hipStream_t s);
+int launch_pf_inv_small(const float* gbuf, int PB, const float* d, const int* perm, int N, int n, int64_t batch,
+                        int adjugate, const float* scale, float* out, hipStream_t s);
+
 // 128 < n <= PF_LARGE_MAXN Parlett-Reid (pf_large.hip); with gbuf the factors
 // (B, N/PB, N, PB) by original row (PB = pf_large_block_cols(N)), d (B, N/2) and perm (B, N).
 constexpr int PF_LARGE_MAXN = 8192;

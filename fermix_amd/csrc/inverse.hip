@@ -1,8 +1,9 @@
-// A^-T from the packed LU of P A' (the slogdet backward), any N: the factors are
-// embedded in T (Ninv x Ninv, Ninv = 32 * 2^k >= N, identity padded) and
-//   1. the 128x128 (or Ninv x Ninv, if smaller) diagonal blocks are inverted in place in
-//      LDS: strictly-lower part of L^-1, upper part of U~^-1 (U~ = U with exact zero
-//      pivots replaced by 1, so singular inputs stay finite);
+// A^-T from the packed LU of P A' (the slogdet backward), N > 128 (smaller orders:
+// small_inverse.hip): the factors are embedded in T (Ninv x Ninv, Ninv = 32 * 2^k >= N,
+// identity padded) and
+//   1. the 128x128 diagonal blocks are inverted in place in LDS: strictly-lower part of
+//      L^-1, upper part of U~^-1 (U~ = U with exact zero pivots replaced by 1, so singular
+//      inputs stay finite);
 //   2. the block-recursive levels s = 128, 256, .., Ninv/2 complete L^-1 and U~^-1 with
 //      four batched MFMA GEMMs per level (all block pairs of a level in one launch):
 //        X21 = -X22 (L21 X11),   Y12 = -Y11 (U12 Y22);
@@ -41,7 +42,7 @@ __device__ __forceinline__ float upper_at(const float* Ts, int ld, int r, int c)
   return r <= c ? Ts[r * ld + c] : 0.0f;
 }
 
-// In-place inverses of the D x D diagonal blocks of the packed T (D = min(128, Ninv)):
+// In-place inverses of the D x D diagonal blocks of the packed T (D = 128):
 // the strictly-lower part becomes L^-1, and with upper the upper part U~^-1, over the
 // whole block, in one workgroup with the block in LDS:
 //   1. the 32x32 leaves by substitution, one wave per leaf: lane c (< 32) forms column c
@@ -220,16 +221,9 @@ __global__ __launch_bounds__(256) void zero_bad_kernel(const int* __restrict__ b
 int launch_tri_inverse(float* T, int Ninv, int64_t batch, float* Tmp, bool upper, hipStream_t s,
                        const int* active, int x3) {
   const int64_t NN = (int64_t)Ninv * Ninv;
-  const int D = Ninv < 128 ? Ninv : 128;  // diagonal blocks inverted whole in LDS
-  if (D == 32)
-    hipLaunchKernelGGL((diag_inverse_kernel<32>), dim3(Ninv / 32, (unsigned)batch), dim3(256), 0, s, T, Ninv, active,
-                       (int)upper);
-  else if (D == 64)
-    hipLaunchKernelGGL((diag_inverse_kernel<64>), dim3(Ninv / 64, (unsigned)batch), dim3(256), 0, s, T, Ninv, active,
-                       (int)upper);
-  else
-    hipLaunchKernelGGL((diag_inverse_kernel<128>), dim3(Ninv / 128, (unsigned)batch), dim3(256), 0, s, T, Ninv,
-                       active, (int)upper);
+  constexpr int D = 128;  // diagonal blocks inverted whole in LDS
+  hipLaunchKernelGGL((diag_inverse_kernel<D>), dim3(Ninv / D, (unsigned)batch), dim3(256), 0, s, T, Ninv, active,
+                     (int)upper);
   if (hipGetLastError() != hipSuccess) return FX_ERR_LAUNCH;
   for (int sz = D; sz < Ninv; sz *= 2) {
     const int pairs = Ninv / (2 * sz);
@@ -337,6 +331,7 @@ int inv_padded(int N) {
 }
 
 size_t lu_inverse_workspace(int64_t batch, int N, bool need_copy) {
+  if (N <= SMALL_INV_MAXN) return ((size_t)batch * 4 + 255) / 256 * 256;  // nominal: nothing is kept there
   const int Ninv = inv_padded(N);
   const int nt = (N + 63) / 64;  // 64x64 tiles of the Z product
   size_t bytes = 0;
@@ -354,6 +349,8 @@ int launch_lu_inverse(float* LU, const int* g0, int N, int n, int64_t batch, con
   const int Ninv = inv_padded(N);
   const bool need_copy = !(in_place && Ninv == N);
   if (!ws || ws_bytes < lu_inverse_workspace(batch, N, need_copy)) return FX_ERR_WORKSPACE;
+  if (N <= SMALL_INV_MAXN)
+    return launch_lu_inv_small(LU, g0, N, n, batch, sign, nullptr, scale, zero_singular, false, invT, s);
   char* p = (char*)ws;
   auto take = [&](size_t x) {
     char* q = p;

@@ -1,5 +1,5 @@
 // S^-1 (inverse mode) or pf(S) S^-1 (adjugate mode) from the forward's own Parlett-Reid
-// factors (the slogpf / pf backward), any N. With P S' P^T = L D L^T, D = diag_s(d_s J),
+// factors (the slogpf / pf backward), N > 128 (smaller orders: small_inverse.hip). With P S' P^T = L D L^T, D = diag_s(d_s J),
 // the pivot K of smallest |d| and d~ = d with d_K and exact zeros replaced by 1:
 //   L~ = L with the a-columns scaled by 1/d~ (unit lower), Y = L~^-1,
 //   DY = rows (Y[p_s], -Y[a_s]) / d~_s,   R = Y^T DY (exactly skew),
@@ -269,6 +269,7 @@ __global__ __launch_bounds__(256) void pf_zero_bad_kernel(const int* __restrict_
 }
 
 size_t pf_inverse_workspace(int64_t batch, int N) {
+  if (N <= SMALL_INV_MAXN) return ((size_t)batch * 4 + 255) / 256 * 256;  // nominal: nothing is kept there
   const int Ninv = inv_padded(N);
   size_t bytes = 0;
   auto add = [&](size_t x) { bytes += (x + 255) / 256 * 256; };
@@ -291,6 +292,8 @@ int launch_pf_inverse(const float* gbuf, int PB, const float* d, const int* perm
                       int x3) {
   const int Ninv = inv_padded(N);
   if (!ws || ws_bytes < pf_inverse_workspace(batch, N)) return FX_ERR_WORKSPACE;
+  if (N <= SMALL_INV_MAXN)
+    return launch_pf_inv_small(gbuf, PB, d, perm, N, n, batch, adjugate, scale, out, s);
   char* p = (char*)ws;
   auto take = [&](size_t x) {
     char* q = p;
