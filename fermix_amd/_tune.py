@@ -6,7 +6,7 @@ The reference's table holds Triton tiles and warps per NVIDIA architecture and d
 kind. The gfx950 table holds the size thresholds of the C library's own dispatch
 decisions (``struct fx_tune`` in include/fermix.h): which kernel family runs an order n,
 whether the blocked LU goes in block pairs, when the Parlett-Reid blocks are 64 columns
-wide, when the GEMMs take 128 x 128 tiles, and the float64 kernels' register limits.
+wide, when the GEMMs take 128 x 128 tiles, and the float64 LDS kernels' limit.
 Every choice is made from n alone, never from the batch size, so batched and vmapped
 calls run the same arithmetic. The C library holds the table (``fx_tune_table``) and
 reads the values in effect on every call; ``TUNES`` below states the same values and a
@@ -136,7 +136,7 @@ class Tune:
     gemm128_x3_min_mn: int = 128
     gemm128_x3_min_k: int = 128
     gemm128_x3_tout: int = 1
-    # float64: registers for n <= f64_reg_max_n, 16-column strips for n <= f64_strip16_max_n
+    # float64: the matrix in LDS for n <= f64_reg_max_n (f64_strip16_max_n: no effect)
     f64_reg_max_n: int = 128
     f64_strip16_max_n: int = 64
     # blocked float32 Parlett-Reid: two halves, one half's panels beside the other half's

@@ -10,19 +10,14 @@
 // Layout: interleaved (re, im) pairs, row-major, batch-major -- the memory of torch's
 // complex64 / complex128 tensors; sign is one complex value per member, logabs real.
 //
-// Kernels (one workgroup of 1024 threads per matrix; the matrix in LDS when it fits in
-// 60 KiB, else in a per-matrix slice of the workspace, served from L2):
-//  - cgj_kernel<F, MODE>: Gauss-Jordan with virtual partial pivoting (the pivot of column
-//    j is the unassigned row of largest |re| + |im|, lowest row on ties), generic over the
-//    field F (cx<float>, cx<double>, and double for the float64 det gradient). GJ_FWD
-//    updates only the unassigned rows (an LU); GJ_INV / GJ_ADJ also the assigned rows and
-//    the identity block [A | I], and row j of A^-1 is row prow[j] of the right block times
-//    the pivot's reciprocal; GJ_ADJ forms det's gradient adj(A)^T from it, continued to
-//    exactly singular A. The element update is the same in every mode, so the gradient
-//    calls give bit-identical sign / logabs;
-//  - cpr_kernel<T>: Parlett-Reid with the pivot row / column swapped into position c + 1,
-//    d = S[c, c+1], tau = -S[:, c] / d, w = S[:, c+1] and the rank-2 update
-//    tau w^T - w tau^T on the rows and columns after c + 1;
+// The values, A^-T and S^-1 come from the LDS-resident kernels of field_small.inc (n <= 128;
+// the LU of complex128 n <= 96) and the blocked kernels of lu64_impl.inc above. Here are the
+// kernels of the adjugates (one workgroup of 1024 threads per matrix; the matrix in LDS when
+// it fits in 60 KiB, else in a per-matrix slice of the workspace, served from L2):
+//  - cgj_kernel<F, MODE>: Gauss-Jordan on [A | I] with virtual partial pivoting (the pivot of
+//    column j is the unassigned row of largest |re| + |im|, lowest row on ties), generic
+//    over the field F = cx<float>, cx<double>, double, float. GJ_ADJ forms det's gradient
+//    adj(A)^T of the exactly singular members from it;
 //  - the Pfaffian adjugate pf(S) S^-1 (pf's gradient) of the float64 and complex kinds:
 //    cpfa_factor_kernel<F> (Parlett-Reid keeping the permutation, the pivots and the
 //    factor column of the smallest pivot) and cgj_kernel<F, GJ_PFA> (the inverse of the
@@ -42,23 +37,9 @@ namespace {
 constexpr int CX_MAXN = 8192;
 constexpr size_t CX_LDS_MAX = 60 * 1024;  // matrix bytes kept in LDS
 constexpr int CX_NT = 1024;
-// complex orders above this run the blocked kernels of lu64_impl.inc (LU, solves, Parlett-Reid
-// with the trailing updates on the fp64 MFMA); up to it, the one-workgroup kernels here
-constexpr int CX_BLK_MIN = 64;
-
-template <class F>
-bool blocked(int n) {
-  return !std::is_same<F, double>::value && n > CX_BLK_MIN;
-}
-
-
-template <class F>
-__device__ __forceinline__ void write_sl(F* sign_out, typename Fd<F>::R* logabs_out, int64_t b, bool singular,
-                                         double2 sgn, double logabs) {
-  using R = typename Fd<F>::R;
-  sign_out[b] = singular ? Fd<F>::zero() : Fd<F>::from(sgn);
-  logabs_out[b] = singular ? R(-INFINITY) : R(logabs);
-}
+// complex orders above this form the Pfaffian adjugate from the LU where it is safe to (the
+// pair pivots' spread); up to it every member takes the pivot-replaced formula
+constexpr int CX_PFA_MAX = 64;
 
 // S (skew != 0: (a - a^T) / 2) into M with row stride ld; with ident, M[:, n:2n] = I.
 
@@ -73,7 +54,7 @@ __device__ __forceinline__ void cload(const F* __restrict__ a, int n, int skew, 
   }
 }
 
-enum { GJ_FWD = 0, GJ_INV = 1, GJ_ADJ = 2, GJ_PFA = 3 };
+enum { GJ_ADJ = 2, GJ_PFA = 3 };
 
 // ---- the Pfaffian adjugate pf(S) S^-1 (the pf gradient) of the 64-bit and complex kinds.
 // Parlett-Reid with the rows and columns permuted (P), P S P^T = L D L^T with D = diag_s(
@@ -119,12 +100,9 @@ PfaLayout pfa_layout(int n) {
   return L;
 }
 
-// Gauss-Jordan on [A | I] (MODE != GJ_FWD) or A. A zero pivot is taken as 1 for the
-// elimination (the U~ convention: its column has no nonzero candidate, so only the
-// assigned rows change), which leaves the forward unchanged and makes the right block
-// X~ = (P^T L U~)^-1 in GJ_ADJ.
-//  - GJ_INV: out = A^-1 (out_t: A^-T), zero for a zero pivot, a zero `gate` value or a
-//    non-finite result;
+// Gauss-Jordan on [A | I]. A zero pivot is taken as 1 for the elimination (the U~
+// convention: its column has no nonzero candidate, so only the assigned rows change), which
+// makes the right block X~ = (P^T L U~)^-1 in GJ_ADJ.
 //  - GJ_ADJ: out = adj(A)^T = d det / dA, from the same pivots: det(A) A^-T when no pivot
 //    is zero; with zero pivots at columns k1 <= ... <= km (km the last) the rank-1
 //    continuation s X~[km, i] X~[j, g(k1)] at (i, j), s = sgn(P) d_K (times
@@ -134,15 +112,13 @@ PfaLayout pfa_layout(int n) {
 //    are zero) and (U~^-1)[k1, km] = X~[k1, g(km)]; a non-finite result gives 0.
 template <class F, int MODE>
 __global__ __launch_bounds__(CX_NT) void cgj_kernel(const F* __restrict__ a, int n, int skew, F* Wg, int use_lds,
-                                                    F* __restrict__ sign_out, typename Fd<F>::R* __restrict__ logabs_out,
-                                                    F* __restrict__ out, int out_t, const F* __restrict__ gate,
+                                                    F* __restrict__ out, const F* __restrict__ gate,
                                                     unsigned char* __restrict__ meta, PfaLayout PL, int eval) {
   using D = Fd<F>;
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ unsigned long long redk[2][CX_NT / 64];
   __shared__ int redr[2][CX_NT / 64];
-  constexpr bool RIGHT = MODE != GJ_FWD;
-  const int ld = RIGHT ? 2 * n : n;
+  const int ld = 2 * n;
   const size_t mat = (size_t)n * ld;
   const int64_t b = blockIdx.x;
   F* M = use_lds ? (F*)smem : Wg + (size_t)b * mat;
@@ -191,7 +167,7 @@ __global__ __launch_bounds__(CX_NT) void cgj_kernel(const F* __restrict__ a, int
     // GJ_ADJ with a gate: only the members whose gate value is 0 (exactly singular ones,
     // the others' adjugate formed by the caller)
     if (MODE == GJ_ADJ && gate && !Fd<F>::is0(gate[b])) return;
-    cload<F>(a + (size_t)b * n * n, n, skew, M, ld, RIGHT);
+    cload<F>(a + (size_t)b * n * n, n, skew, M, ld, true);
   }
   for (int r = threadIdx.x; r < n; r += CX_NT) asg[r] = 0;
   __syncthreads();
@@ -223,7 +199,7 @@ __global__ __launch_bounds__(CX_NT) void cgj_kernel(const F* __restrict__ a, int
     }
     const F* P = M + (size_t)p * ld;
     for (int r = wave; r < n; r += CX_NT / 64) {
-      if (r == p || (!RIGHT && asg[r])) continue;
+      if (r == p) continue;
       F* R = M + (size_t)r * ld;
       const F l = D::mul(R[j], rinv);
       for (int c = j + 1 + lane; c < ld; c += 64) R[c] = D::fms(R[c], l, P[c]);
@@ -279,27 +255,7 @@ __global__ __launch_bounds__(CX_NT) void cgj_kernel(const F* __restrict__ a, int
       ++cycles;
       for (int t = s; !asg[t]; t = prow[t]) asg[t] = 1;
     }
-    const bool odd = (n - cycles) & 1;
-    write_sl<F>(sign_out, logabs_out, b, nzero > 0, odd ? make_double2(-sgn.x, -sgn.y) : sgn, logabs);
-    if (MODE == GJ_ADJ) redk[0][0] = odd ? 1ull : 0ull;
-  }
-  if constexpr (MODE == GJ_INV) {
-    F* O = out + (size_t)b * n * n;
-    const bool zero = nzero > 0 || (gate && D::is0(gate[b]));
-    bool bad = false;
-    if (!zero) {
-      // A^-1[j, c] = M[prow[j], n + c] / pivot_j; out_t: O[c, j], else O[j, c]
-      for (int e = threadIdx.x; e < n * n; e += CX_NT) {
-        const int r = e / n, q = e - r * n;
-        const int j = out_t ? q : r, c = out_t ? r : q;
-        const F* Pj = M + (size_t)prow[j] * ld;
-        const F v = D::mul(Pj[n + c], D::rcp(Pj[j]));
-        bad |= !D::finite(v);
-        O[e] = v;
-      }
-    }
-    if (zero || __syncthreads_or(bad))
-      for (int e = threadIdx.x; e < n * n; e += CX_NT) O[e] = D::zero();
+    redk[0][0] = (n - cycles) & 1 ? 1ull : 0ull;
   }
   if constexpr (MODE == GJ_ADJ) {
     __syncthreads();
@@ -339,80 +295,9 @@ __global__ __launch_bounds__(CX_NT) void cgj_kernel(const F* __restrict__ a, int
   }
 }
 
-template <class T>
-__global__ __launch_bounds__(CX_NT) void cpr_kernel(const cx<T>* __restrict__ a, int n, int skew, cx<T>* Wg,
-                                                    int use_lds, cx<T>* __restrict__ sign_out,
-                                                    T* __restrict__ logabs_out) {
-  using F = cx<T>;
-  using D = Fd<F>;
-  extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ unsigned long long redk[2][CX_NT / 64];
-  __shared__ int redr[2][CX_NT / 64];
-  const size_t mat = (size_t)n * n;
-  const int64_t b = blockIdx.x;
-  if (n & 1) {  // odd n: pf = 0
-    if (threadIdx.x == 0) write_sl<F>(sign_out, logabs_out, b, true, make_double2(0.0, 0.0), 0.0);
-    return;
-  }
-  F* M = use_lds ? (F*)smem : Wg + (size_t)b * mat;
-  cload<F>(a + (size_t)b * mat, n, skew, M, n, false);
-  __syncthreads();
-
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  double logabs = 0.0;
-  double2 sgn = make_double2(1.0, 0.0);
-  bool singular = false;
-  for (int c = 0; c + 1 < n; c += 2) {
-    unsigned long long k = 0;
-    int row = 0x7fffffff;
-    // |S[r, c]| = |S[c, r]|: the candidates read along row c
-    for (int r = c + 1 + threadIdx.x; r < n; r += CX_NT) take_better(k, row, D::key(M[(size_t)c * n + r]), r);
-    const int p = block_argmax<CX_NT>(k, row, redk[(c >> 1) & 1], redr[(c >> 1) & 1]);
-    const int q = c + 1;
-    if (p != q) {  // swap rows p, q over columns >= c, then columns p, q over rows >= c
-      sgn = make_double2(-sgn.x, -sgn.y);
-      for (int x = c + threadIdx.x; x < n; x += CX_NT) {
-        const F u = M[(size_t)p * n + x], v = M[(size_t)q * n + x];
-        M[(size_t)p * n + x] = v;
-        M[(size_t)q * n + x] = u;
-      }
-      __syncthreads();
-      for (int x = c + threadIdx.x; x < n; x += CX_NT) {
-        const F u = M[(size_t)x * n + p], v = M[(size_t)x * n + q];
-        M[(size_t)x * n + p] = v;
-        M[(size_t)x * n + q] = u;
-      }
-      __syncthreads();
-    }
-    const F d = M[(size_t)c * n + q];
-    if (D::is0(d)) {
-      singular = true;
-      break;
-    }
-    D::acc(sgn, logabs, d);
-    const F rd = D::rcp(d);
-    // tau = -S[:, c] / d = S[c, :] / d, w = S[:, q] = -S[q, :] (rows c and q contiguous);
-    // S[r, x] += tau_r w_x - w_r tau_x
-    const F* Rc = M + (size_t)c * n;
-    const F* Rq = M + (size_t)q * n;
-    for (int r = q + 1 + wave; r < n; r += CX_NT / 64) {
-      F* R = M + (size_t)r * n;
-      const F tr = D::mul(Rc[r], rd);
-      const F wr = {-Rq[r].re, -Rq[r].im};
-      for (int x = q + 1 + lane; x < n; x += 64) {
-        const F wx = {-Rq[x].re, -Rq[x].im};
-        const F tx = D::mul(Rc[x], rd);
-        const F t1 = D::mul(tr, wx), t2 = D::mul(wr, tx);
-        R[x] = F{R[x].re + (t1.re - t2.re), R[x].im + (t1.im - t2.im)};
-      }
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) write_sl<F>(sign_out, logabs_out, b, singular, sgn, logabs);
-}
-
-// Parlett-Reid of the Pfaffian adjugate (any field): the pair steps of cpr_kernel with
-// whole rows swapped (so the factor's columns below each pair, which the L~ formula reads,
+// Parlett-Reid of the Pfaffian adjugate (any field): the pivot row / column swapped into
+// position c + 1, d = S[c, c+1], tau = -S[:, c] / d, w = S[:, c+1] and the rank-2 update tau
+// w^T - w tau^T on the rows and columns after c + 1, with whole rows swapped (so the factor's columns below each pair, which the L~ formula reads,
 // move with the permutation), the permutation kept, and no stop at a zero pivot (tau = 0
 // there: the step changes nothing, as in the reference's masked step). Thread 0 keeps the
 // pivot statistics; the end writes the member's PfaHead, the permutation, d and
@@ -581,38 +466,15 @@ constexpr int max_n() {
   return sizeof(F) == 4 ? GEN32_MAXN : CX_MAXN;
 }
 
+// adj(A)^T of the members whose gate value is 0 (exactly singular ones) into out.
 template <class F>
-int launch_cgj(const void* a, int n, int skew, int64_t batch, void* sign, void* logabs, void* out, int mode,
-               int out_t, const void* gate, void* ws, size_t ws_bytes, hipStream_t s) {
-  using R = typename Kind<F>::R;
-  const int ld = mode != GJ_FWD ? 2 * n : n;
-  const bool lds = cx_in_lds<F>(n, ld);
-  if (!lds && (!ws || ws_bytes < cx_matrix_ws<F>(batch, n, ld))) return FX_ERR_WORKSPACE;
-  const size_t shm = cx_lds_bytes((size_t)n * ld * sizeof(F), n, lds, true);
-  const dim3 grid((unsigned)batch);
-  const F* A = (const F*)a;
-  F* W = (F*)ws;
-  F* sg = (F*)sign;
-  R* lg = (R*)logabs;
-  if (mode == GJ_INV)
-    cgj_kernel<F, GJ_INV><<<grid, CX_NT, shm, s>>>(A, n, skew, W, lds, sg, lg, (F*)out, out_t, (const F*)gate, nullptr, PfaLayout{}, 0);
-  else if (mode == GJ_ADJ)
-    cgj_kernel<F, GJ_ADJ><<<grid, CX_NT, shm, s>>>(A, n, skew, W, lds, sg, lg, (F*)out, 1, (const F*)gate, nullptr,
-                                                   PfaLayout{}, 0);
-  else
-    cgj_kernel<F, GJ_FWD><<<grid, CX_NT, shm, s>>>(A, n, skew, W, lds, sg, lg, nullptr, 0, nullptr, nullptr,
-                                                  PfaLayout{}, 0);
-  return hipGetLastError() == hipSuccess ? FX_OK : FX_ERR_LAUNCH;
-}
-
-template <class T>
-int launch_cpr(const void* a, int n, int skew, int64_t batch, void* sign, void* logabs, void* ws, size_t ws_bytes,
-               hipStream_t s) {
-  using F = cx<T>;
-  const bool lds = cx_in_lds<F>(n, n);
-  if (!lds && (!ws || ws_bytes < cx_matrix_ws<F>(batch, n, n))) return FX_ERR_WORKSPACE;
-  const size_t shm = cx_lds_bytes((size_t)n * n * sizeof(F), n, lds, false);
-  cpr_kernel<T><<<dim3((unsigned)batch), CX_NT, shm, s>>>((const F*)a, n, skew, (F*)ws, lds, (F*)sign, (T*)logabs);
+int launch_singular_adjugate(const F* A, int n, int64_t batch, F* out, const F* gate, void* ws, size_t ws_bytes,
+                             hipStream_t s) {
+  const bool lds = cx_in_lds<F>(n, 2 * n);
+  if (!lds && (!ws || ws_bytes < cx_matrix_ws<F>(batch, n, 2 * n))) return FX_ERR_WORKSPACE;
+  const size_t shm = cx_lds_bytes((size_t)n * 2 * n * sizeof(F), n, lds, true);
+  cgj_kernel<F, GJ_ADJ><<<dim3((unsigned)batch), CX_NT, shm, s>>>(A, n, 0, (F*)ws, lds, out, gate, nullptr,
+                                                                 PfaLayout{}, 0);
   return hipGetLastError() == hipSuccess ? FX_OK : FX_ERR_LAUNCH;
 }
 
@@ -649,23 +511,72 @@ int cx_empty(void* sign, void* logabs, int64_t batch, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? FX_OK : FX_ERR_LAUNCH;
 }
 
+// The LU (values; with the inverse) and the Parlett-Reid of a field: the matrix in LDS where
+// field_small.inc covers the order (no workspace), else the blocked kernels. The orders
+// follow from what 160 KiB hold. Measured, us, slogdet / + gradient / slogpf / + gradient:
+//   complex64  B = 1024, n = 64   853 / 1256 / 435 / 1701 -> 48 / 147 / 49 / 212
+//   complex64  B = 1024, n = 100  915 / 1791 / 1192 / 3040 -> 465 / 623 / 264 / 917
+//   complex128 B = 1024, n = 64   1311 / 1857 / 744 / 2621 -> 113 / 207 / 99 / 321
+//   complex128 B = 1024, n = 96   1189 / 2039 / 1488 / 3576 -> 529 / 718 / 387 / 1126
+// (before: one unblocked workgroup of 1024 threads for n <= 64, the blocked kernels above).
+template <class F>
+bool lds_lu(int n) {
+  if constexpr (std::is_same<F, float>::value) return false;
+  else return fsmall_lu_covers<F>(n);
+}
+template <class F>
+bool lds_pr(int n) {
+  if constexpr (std::is_same<F, float>::value) return false;
+  else return fsmall_pr_covers<F>(n);
+}
+template <class F>
+size_t lu_ws(int64_t batch, int n) {
+  return lds_lu<F>(n) ? 0 : blk_lu_workspace<F>(batch, n);
+}
+template <class F>
+size_t lu_inverse_ws(int64_t batch, int n) {
+  return lds_lu<F>(n) ? 0 : blk_lu_inverse_workspace<F>(batch, n);
+}
+template <class F>
+size_t pr_ws(int64_t batch, int n) {
+  return lds_pr<F>(n) ? 0 : blk_pr_workspace<F>(batch, n);
+}
+template <class F>
+int lu_values(const F* a, int n, int64_t batch, F* sign, typename Fd<F>::R* logabs, void* ws, size_t wsb,
+              hipStream_t s) {
+  if constexpr (!std::is_same<F, float>::value)
+    if (lds_lu<F>(n)) return fsmall_lu<F>(a, n, 0, batch, sign, logabs, nullptr, nullptr, nullptr, nullptr, 0, s);
+  return blk_lu<F>(a, n, batch, sign, logabs, ws, wsb, s);
+}
+template <class F>
+int lu_inverse(const F* a, int n, int skew, int64_t batch, F* sign, typename Fd<F>::R* logabs, const F* gate,
+               const F* ssign, const typename Fd<F>::R* slog, F* out, int out_t, void* ws, size_t wsb, hipStream_t s) {
+  if constexpr (!std::is_same<F, float>::value)
+    if (lds_lu<F>(n)) return fsmall_lu<F>(a, n, skew, batch, sign, logabs, gate, ssign, slog, out, out_t, s);
+  return blk_lu_inverse<F>(a, n, skew, batch, sign, logabs, gate, ssign, slog, out, out_t, ws, wsb, s);
+}
+template <class F>
+int pr_values(const F* a, int n, int skew, int64_t batch, F* sign, typename Fd<F>::R* logabs, void* ws, size_t wsb,
+              hipStream_t s, double* spread = nullptr) {
+  if constexpr (!std::is_same<F, float>::value)
+    if (lds_pr<F>(n)) return fsmall_pr<F>(a, n, skew, batch, sign, logabs, s, spread);
+  return blk_pr<F>(a, n, skew, batch, sign, logabs, ws, wsb, s, spread);
+}
+
 template <class F>
 size_t slogdet_ws(int64_t batch, int n) {
-  if (n > max_n<F>()) return 0;
-  return blocked<F>(n) ? blk_lu_workspace<F>(batch, n) : cx_matrix_ws<F>(batch, n, n);
+  return n > max_n<F>() ? 0 : lu_ws<F>(batch, n);
 }
 template <class F>
 size_t slogdet_parts_ws(int64_t batch, int n) {
-  if (n > max_n<F>()) return 0;
-  return blocked<F>(n) ? blk_lu_inverse_workspace<F>(batch, n) : cx_matrix_ws<F>(batch, n, 2 * n);
+  return n > max_n<F>() ? 0 : lu_inverse_ws<F>(batch, n);
 }
-// det's gradient: blocked, the LU solves plus the Gauss-Jordan run for the singular members
-// (its [A | I] and its sign / logabs in scratch)
+// det's gradient: the LU's inverse plus the Gauss-Jordan run for the singular members
+// (its [A | I])
 template <class F>
 size_t det_parts_ws(int64_t batch, int n) {
-  if (n > max_n<F>() || !blocked<F>(n) || batch <= 0) return slogdet_parts_ws<F>(batch, n);
-  return align_up(blk_lu_inverse_workspace<F>(batch, n)) + align_up(cx_matrix_ws<F>(batch, n, 2 * n)) +
-         align_up((size_t)batch * 2 * sizeof(F));
+  if (n > max_n<F>() || batch <= 0) return 0;
+  return align_up(lu_inverse_ws<F>(batch, n)) + align_up(cx_matrix_ws<F>(batch, n, 2 * n));
 }
 
 template <class F>
@@ -674,8 +585,7 @@ int slogdet(const void* a, int64_t batch, int n, void* sign, void* logabs, void*
   if (st != FX_OK || batch == 0) return st;
   if (n == 0) return cx_empty<F>(sign, logabs, batch, s);
   using R = typename Kind<F>::R;
-  if (blocked<F>(n)) return blk_lu<F>((const F*)a, n, batch, (F*)sign, (R*)logabs, ws, wsb, s);
-  return launch_cgj<F>(a, n, 0, batch, sign, logabs, nullptr, GJ_FWD, 0, nullptr, ws, wsb, s);
+  return lu_values<F>((const F*)a, n, batch, (F*)sign, (R*)logabs, ws, wsb, s);
 }
 
 template <class F>
@@ -685,13 +595,9 @@ int slogdet_parts(const void* a, int64_t batch, int n, void* sign, void* logabs,
   if (st != FX_OK || batch == 0) return st;
   if (n == 0) return cx_empty<F>(sign, logabs, batch, s);
   using R = typename Kind<F>::R;
-  if (blocked<F>(n)) {
-    if (!inv_t) return blk_lu<F>((const F*)a, n, batch, (F*)sign, (R*)logabs, ws, wsb, s);
-    return blk_lu_inverse<F>((const F*)a, n, 0, batch, (F*)sign, (R*)logabs, nullptr, nullptr, nullptr, (F*)inv_t, 1,
-                             ws, wsb, s);
-  }
-  if (!inv_t) return launch_cgj<F>(a, n, 0, batch, sign, logabs, nullptr, GJ_FWD, 0, nullptr, ws, wsb, s);
-  return launch_cgj<F>(a, n, 0, batch, sign, logabs, inv_t, GJ_INV, 1, nullptr, ws, wsb, s);
+  if (!inv_t) return lu_values<F>((const F*)a, n, batch, (F*)sign, (R*)logabs, ws, wsb, s);
+  return lu_inverse<F>((const F*)a, n, 0, batch, (F*)sign, (R*)logabs, nullptr, nullptr, nullptr, (F*)inv_t, 1, ws,
+                       wsb, s);
 }
 
 // det's gradient adj(A)^T with sign / logabs of the same run
@@ -702,58 +608,47 @@ int det_parts(const void* a, int64_t batch, int n, void* sign, void* logabs, voi
   if (st != FX_OK || batch == 0) return st;
   if (n > 0 && !adj_t) return FX_ERR_INVALID_ARGUMENT;
   if (n == 0) return cx_empty<F>(sign, logabs, batch, s);
-  if (blocked<F>(n)) {  // as det_parts_f64 below: the regular members from the LU solves
-    using R = typename Kind<F>::R;
-    if (!ws || wsb < det_parts_ws<F>(batch, n)) return FX_ERR_WORKSPACE;
-    const size_t lw = align_up(blk_lu_inverse_workspace<F>(batch, n)), gw = align_up(cx_matrix_ws<F>(batch, n, 2 * n));
-    char* base = (char*)ws;
-    const int r = blk_lu_inverse<F>((const F*)a, n, 0, batch, (F*)sign, (R*)logabs, nullptr, (const F*)sign,
-                                    (const R*)logabs, (F*)adj_t, 1, base, lw, s);
-    if (r != FX_OK) return r;
-    F* gsign = (F*)(base + lw + gw);
-    return launch_cgj<F>(a, n, 0, batch, gsign, gsign + batch, adj_t, GJ_ADJ, 1, sign, base + lw, gw, s);
-  }
-  return launch_cgj<F>(a, n, 0, batch, sign, logabs, adj_t, GJ_ADJ, 1, nullptr, ws, wsb, s);
+  // sign / logabs (the forward's bits) and the regular members' det(A) A^-T from the LU, the
+  // exactly singular members' from a Gauss-Jordan run gated to them
+  using R = typename Kind<F>::R;
+  const size_t need = det_parts_ws<F>(batch, n);
+  if (need && (!ws || wsb < need)) return FX_ERR_WORKSPACE;
+  const size_t lw = align_up(lu_inverse_ws<F>(batch, n)), gw = align_up(cx_matrix_ws<F>(batch, n, 2 * n));
+  char* base = (char*)ws;
+  const int r = lu_inverse<F>((const F*)a, n, 0, batch, (F*)sign, (R*)logabs, nullptr, (const F*)sign,
+                              (const R*)logabs, (F*)adj_t, 1, base, lw, s);
+  if (r != FX_OK) return r;
+  return launch_singular_adjugate<F>((const F*)a, n, batch, (F*)adj_t, (const F*)sign, base + lw, gw, s);
 }
 
-// float64 above the register kernels' orders: sign / logabs (the forward's bits) and the
-// regular members' adjugate det(A) A^-T from the blocked LU and its solves, the exactly
-// singular members' from a Gauss-Jordan run gated to them (its values in scratch).
+// float64: the same, with the LU above f64_reg_max_n the blocked one.
 size_t det_parts_f64_ws(int64_t batch, int n) {
   if (n > CX_MAXN || batch <= 0) return 0;
-  if (n <= tune().f64_reg_max_n) return slogdet_parts_ws<double>(batch, n);
-  return align_up(lu64_inverse_workspace(batch, n)) + align_up(slogdet_parts_ws<double>(batch, n)) +
-         align_up((size_t)batch * 2 * sizeof(double));
+  const bool lds = n <= tune().f64_reg_max_n;
+  return (lds ? 0 : align_up(lu64_inverse_workspace(batch, n))) + align_up(cx_matrix_ws<double>(batch, n, 2 * n));
 }
 
 int det_parts_f64(const double* a, int64_t batch, int n, double* sign, double* logabs, double* adj_t, void* ws,
                   size_t wsb, hipStream_t s) {
-  if (n <= tune().f64_reg_max_n) return det_parts<double>(a, batch, n, sign, logabs, adj_t, ws, wsb, s);
   const int st = check_cx_args<double>(a, batch, n, sign, logabs, adj_t, ws);
   if (st != FX_OK || batch == 0) return st;
-  if (!adj_t) return FX_ERR_INVALID_ARGUMENT;
+  if (n > 0 && !adj_t) return FX_ERR_INVALID_ARGUMENT;
+  if (n == 0) return cx_empty<double>(sign, logabs, batch, s);
   const size_t need = det_parts_f64_ws(batch, n);
-  if (!ws || wsb < need) return FX_ERR_WORKSPACE;
-  const size_t lw = align_up(lu64_inverse_workspace(batch, n)), gw = align_up(slogdet_parts_ws<double>(batch, n));
+  if (need && (!ws || wsb < need)) return FX_ERR_WORKSPACE;
+  const bool lds = n <= tune().f64_reg_max_n;
+  const size_t lw = lds ? 0 : align_up(lu64_inverse_workspace(batch, n));
+  const size_t gw = align_up(cx_matrix_ws<double>(batch, n, 2 * n));
   char* base = (char*)ws;
-  const int r = launch_lu64_inverse(a, n, 0, batch, sign, logabs, nullptr, sign, logabs, adj_t, 1, base, lw, s);
+  const int r = lds ? launch_lu64_small(a, n, batch, sign, logabs, adj_t, true, s)
+                    : launch_lu64_inverse(a, n, 0, batch, sign, logabs, nullptr, sign, logabs, adj_t, 1, base, lw, s);
   if (r != FX_OK) return r;
-  double* gsign = (double*)(base + lw + gw);
-  return launch_cgj<double>(a, n, 0, batch, gsign, gsign + batch, adj_t, GJ_ADJ, 1, sign, base + lw, gw, s);
+  return launch_singular_adjugate<double>(a, n, batch, adj_t, sign, base + lw, gw, s);
 }
 
 template <class T>
 size_t slogpf_ws(int64_t batch, int n) {
-  if (n > CX_MAXN) return 0;
-  return blocked<cx<T>>(n) ? blk_pr_workspace<cx<T>>(batch, n) : cx_matrix_ws<cx<T>>(batch, n, n);
-}
-
-template <class T>
-int launch_pf(const T* a, int n, int skew, int64_t batch, T* sign, T* logabs, void* ws, size_t wsb, hipStream_t s,
-              double* spread = nullptr) {
-  if (blocked<cx<T>>(n))
-    return blk_pr<cx<T>>((const cx<T>*)a, n, skew, batch, (cx<T>*)sign, logabs, ws, wsb, s, spread);
-  return launch_cpr<T>(a, n, skew, batch, sign, logabs, ws, wsb, s);
+  return n > CX_MAXN ? 0 : pr_ws<cx<T>>(batch, n);
 }
 
 // The blocked Pfaffian adjugate takes pf(S) S^-1 from an LU of S scaled by the
@@ -833,13 +728,13 @@ int pf_adjugate(const F* a, int64_t batch, int n, int skew, F* g, void* ws, size
   const bool lds = cx_in_lds<F>(n, 2 * n);
   const size_t shm = cx_lds_bytes((size_t)n * 2 * n * sizeof(F), n, lds, true);
   for (int ev = 0; ev < 2; ++ev) {
-    cgj_kernel<F, GJ_PFA><<<grid, CX_NT, shm, s>>>(a, n, skew, W, lds, nullptr, nullptr, g, 0, gate, meta, PL, ev);
+    cgj_kernel<F, GJ_PFA><<<grid, CX_NT, shm, s>>>(a, n, skew, W, lds, g, gate, meta, PL, ev);
     if (hipGetLastError() != hipSuccess) return FX_ERR_LAUNCH;
   }
   return FX_OK;
 }
 
-// The blocked parts run of a field (complex above CX_BLK_MIN, float32 above its own
+// The parts run of a field (complex above CX_PFA_MAX, float32 above its own
 // blocked kernels): the blocked Parlett-Reid for sign / logabs and the pair pivots'
 // spread, then g: S^-1 from the blocked LU solves of the same S (zero where pf = 0), or the
 // Pfaffian adjugate pf(S) S^-1 -- from the same solves scaled by the Parlett-Reid pf for
@@ -850,13 +745,13 @@ int pf_adjugate(const F* a, int64_t batch, int n, int skew, F* g, void* ws, size
 template <class F>
 size_t blk_pf_parts_body(int64_t batch, int n) {
   using R = typename Fd<F>::R;
-  return std::max(align_up(blk_lu_inverse_workspace<F>(batch, n)) + align_up((size_t)batch * (sizeof(F) + sizeof(R))),
+  return std::max(align_up(lu_inverse_ws<F>(batch, n)) + align_up((size_t)batch * (sizeof(F) + sizeof(R))),
                   pf_adjugate_ws<F>(batch, n));
 }
 template <class F>
 size_t blk_pf_parts_ws(int64_t batch, int n) {
   if (batch <= 0 || n <= 0 || n > max_n<F>()) return 0;
-  return align_up(blk_pr_workspace<F>(batch, n)) + blk_pf_parts_body<F>(batch, n) +
+  return align_up(pr_ws<F>(batch, n)) + blk_pf_parts_body<F>(batch, n) +
          align_up((size_t)batch * sizeof(double)) + align_up((size_t)batch * sizeof(F));
 }
 template <class F>
@@ -864,13 +759,13 @@ int blk_pf_parts(const F* A, int64_t batch, int n, int skew, int adjugate, F* si
                  void* ws, size_t wsb, hipStream_t s) {
   using R = typename Fd<F>::R;
   if (!ws || wsb < blk_pf_parts_ws<F>(batch, n)) return FX_ERR_WORKSPACE;
-  const size_t pr = align_up(blk_pr_workspace<F>(batch, n));
+  const size_t pr = align_up(pr_ws<F>(batch, n));
   const size_t body = blk_pf_parts_body<F>(batch, n);
-  const size_t lw = align_up(blk_lu_inverse_workspace<F>(batch, n));
+  const size_t lw = align_up(lu_inverse_ws<F>(batch, n));
   char* base = (char*)ws;
   double* spread = (double*)(base + pr + body);
   F* gz = (F*)(base + pr + body + align_up((size_t)batch * sizeof(double)));
-  int st = blk_pr<F>(A, n, skew, batch, sign, logabs, base, pr, s, spread);
+  int st = pr_values<F>(A, n, skew, batch, sign, logabs, base, pr, s, spread);
   if (st != FX_OK) return st;
   if (adjugate && (n & 1)) return cx_zero<F>(g, batch * (int64_t)n * n, s);
   F* gsign = (F*)(base + pr + lw);
@@ -881,8 +776,8 @@ int blk_pf_parts(const F* A, int64_t batch, int n, int skew, int adjugate, F* si
     if (st != FX_OK) return st;
     gate = gz;
   }
-  st = blk_lu_inverse<F>(A, n, skew, batch, gsign, glog, gate, adjugate ? sign : nullptr, adjugate ? logabs : nullptr,
-                         g, 0, base + pr, lw, s);
+  st = lu_inverse<F>(A, n, skew, batch, gsign, glog, gate, adjugate ? sign : nullptr, adjugate ? logabs : nullptr, g, 0,
+                     base + pr, lw, s);
   if (st != FX_OK || !adjugate) return st;
   return pf_adjugate<F>(A, batch, n, skew, g, base + pr, body, s, gate);
 }
@@ -890,9 +785,9 @@ int blk_pf_parts(const F* A, int64_t batch, int n, int skew, int adjugate, F* si
 template <class T>
 size_t slogpf_parts_ws(int64_t batch, int n) {
   if (n > CX_MAXN || batch <= 0) return 0;
-  if (blocked<cx<T>>(n)) return blk_pf_parts_ws<cx<T>>(batch, n);
-  const size_t inv = align_up(cx_matrix_ws<cx<T>>(batch, n, 2 * n)) + align_up((size_t)batch * 3 * sizeof(T));
-  return align_up(slogpf_ws<T>(batch, n)) + std::max(inv, pf_adjugate_ws<cx<T>>(batch, n));
+  if (n > CX_PFA_MAX) return blk_pf_parts_ws<cx<T>>(batch, n);
+  const size_t inv = align_up((size_t)batch * 3 * sizeof(T));  // the LU run's sign / logabs
+  return std::max(inv, pf_adjugate_ws<cx<T>>(batch, n));
 }
 
 template <class T>
@@ -900,10 +795,10 @@ int slogpf(const T* a, int64_t batch, int n, int skew, T* sign, T* logabs, void*
   const int st = check_cx_args<cx<T>>(a, batch, n, sign, logabs, nullptr, ws);
   if (st != FX_OK || batch == 0) return st;
   if (n == 0) return cx_empty<cx<T>>(sign, logabs, batch, s);
-  return launch_pf<T>(a, n, skew != 0, batch, sign, logabs, ws, wsb, s);
+  return pr_values<cx<T>>((const cx<T>*)a, n, skew != 0, batch, (cx<T>*)sign, logabs, ws, wsb, s);
 }
 
-// The Parlett-Reid run for sign / logabs, then g: S^-1 by Gauss-Jordan on the same S
+// The Parlett-Reid run for sign / logabs, then g: S^-1 from the LU of the same S
 // (zeroed where the Parlett-Reid run found pf = 0; every member for odd n), or the
 // Pfaffian adjugate pf(S) S^-1 (zero for odd n).
 template <class T>
@@ -913,21 +808,18 @@ int slogpf_parts(const T* a, int64_t batch, int n, int skew, int adjugate, T* si
   if (st != FX_OK || batch == 0) return st;
   if (!g) return slogpf<T>(a, batch, n, skew, sign, logabs, ws, wsb, s);
   if (n == 0) return cx_empty<cx<T>>(sign, logabs, batch, s);
-  if (blocked<cx<T>>(n))
+  if (n > CX_PFA_MAX)
     return blk_pf_parts<cx<T>>((const cx<T>*)a, batch, n, skew != 0, adjugate, (cx<T>*)sign, logabs, (cx<T>*)g, ws,
                                wsb, s);
   if (wsb < slogpf_parts_ws<T>(batch, n) || (!ws && slogpf_parts_ws<T>(batch, n))) return FX_ERR_WORKSPACE;
-  const size_t pr = align_up(slogpf_ws<T>(batch, n));
-  char* base = (char*)ws;
-  st = launch_pf<T>(a, n, skew != 0, batch, sign, logabs, base, pr, s);
+  st = pr_values<cx<T>>((const cx<T>*)a, n, skew != 0, batch, (cx<T>*)sign, logabs, nullptr, 0, s);
   if (st != FX_OK) return st;
   if (adjugate && (n & 1)) return cx_zero<cx<T>>((cx<T>*)g, batch * (int64_t)n * n, s);
-  if (adjugate)
-    return pf_adjugate<cx<T>>((const cx<T>*)a, batch, n, skew != 0, (cx<T>*)g, base + pr, wsb - pr, s);
-  const size_t gj = align_up(cx_matrix_ws<cx<T>>(batch, n, 2 * n));
-  T* gsign = (T*)(base + pr + gj);
+  if (adjugate) return pf_adjugate<cx<T>>((const cx<T>*)a, batch, n, skew != 0, (cx<T>*)g, ws, wsb, s);
+  T* gsign = (T*)ws;
   T* glog = gsign + 2 * batch;
-  return launch_cgj<cx<T>>(a, n, skew != 0, batch, gsign, glog, g, GJ_INV, 0, sign, base + pr, gj, s);
+  return lu_inverse<cx<T>>((const cx<T>*)a, n, skew != 0, batch, (cx<T>*)gsign, glog, (const cx<T>*)sign, nullptr,
+                           nullptr, (cx<T>*)g, 0, nullptr, 0, s);
 }
 
 }  // namespace

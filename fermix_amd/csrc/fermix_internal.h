@@ -196,6 +196,10 @@ struct GemmDesc {
 // C = alpha op(A) op(B) + beta C for every (batch, second-batch) index.
 int launch_gemm(const GemmDesc& d, int64_t batch, int nb2, hipStream_t s);
 
+// float64 n <= fx_tune.f64_reg_max_n (f64.hip): sign / logabs and, with out, A^-T (times the
+// determinant with det), zero for singular members
+int launch_lu64_small(const double* a, int n, int64_t batch, double* sign, double* logabs, double* out, bool det,
+                      hipStream_t s);
 // float64 blocked LU (sign, logabs) for the orders above the register kernels (lu64_impl.inc)
 size_t lu64_workspace(int64_t batch, int n);
 int launch_lu64(const double* A, int n, int64_t batch, double* sign, double* logabs, void* ws, size_t ws_bytes,

@@ -159,4 +159,19 @@ template <class F>
 int blk_pr(const F* A, int n, int skew, int64_t batch, F* sign, typename Fd<F>::R* logabs, void* ws, size_t ws_bytes,
            hipStream_t s, double* spread = nullptr);
 
+// The same with the whole matrix in LDS (field_small.inc; no workspace), F = double, cx<float>,
+// cx<double>: covers() is the range of orders (n = 0 included). fsmall_lu without out forms
+// sign / logabs alone, with the bits of the call that also forms out; ssign == sign scales
+// by the factorisation's own det.
+template <class F>
+bool fsmall_lu_covers(int n);
+template <class F>
+bool fsmall_pr_covers(int n);
+template <class F>
+int fsmall_lu(const F* A, int n, int skew, int64_t batch, F* sign, typename Fd<F>::R* logabs, const F* gate,
+              const F* ssign, const typename Fd<F>::R* slog, F* out, int out_t, hipStream_t s);
+template <class F>
+int fsmall_pr(const F* A, int n, int skew, int64_t batch, F* sign, typename Fd<F>::R* logabs, hipStream_t s,
+              double* spread = nullptr);
+
 }  // namespace fx

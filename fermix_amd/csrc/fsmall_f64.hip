@@ -1,0 +1,6 @@
+// The LDS-resident LU / inverse and Parlett-Reid of field_small.inc for double.
+#include "field_small.inc"
+
+namespace fx {
+FSMALL_INSTANTIATE(double)
+}  // namespace fx

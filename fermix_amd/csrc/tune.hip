@@ -24,9 +24,11 @@
 //    operand once into LDS planes, wins on every product from 128 on: slogdet fwd + grad
 //    n = 512 6.32 -> 5.78 ms, n = 1024 9.74 -> 8.64, n = 2048 19.68 -> 17.64, n = 256
 //    4.56 -> 4.41; slogpf fwd + grad 1-4 %;
-//  - f64_reg_max_n 128 / f64_strip16_max_n 64: float64 matrices in registers for
-//    n <= 128 (slogdet n = 128 8.66 -> 3.16 ms against the LDS kernel), in 16-column strips
-//    for n <= 64 (n = 64 1.37 ms; at n = 128 they lose, 3.97 against 3.16 ms);
+//  - f64_reg_max_n 128: float64 in the one-launch kernels (the matrix in LDS) for n <= 128,
+//    the most that 160 KiB hold: B = 1024, n = 128 slogdet 373 us, + A^-T 505, slogpf 230,
+//    + S^-1 775 against 829 / 1800 / 601 / 2490 for the register kernels they replaced and
+//    about the same for the blocked ones. f64_strip16_max_n: those kernels' strip width,
+//    without effect since;
 //  - pf_overlap_max_half 32 / pf_overlap_min_work 256: the Parlett-Reid halves with one
 //    half's panels beside the other's update gain where half an update takes about as
 //    long as a panel (slogpf B = 64, n = 2048 9.06 -> 8.76 ms; B = 16, n = 4096 28.5 ->

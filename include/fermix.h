@@ -131,9 +131,9 @@ typedef struct fx_tune {
   int32_t gemm128_x3_min_mn;
   int32_t gemm128_x3_min_k;
   int32_t gemm128_x3_tout;
-  /* float64: the matrix in registers for n <= f64_reg_max_n (0 .. 128), with rows split
-   * in 16-column strips for n <= f64_strip16_max_n (0 .. 64) and 32-column ones above;
-   * larger n runs one workgroup per matrix in LDS or in the workspace */
+  /* float64: one launch with the matrix in LDS for n <= f64_reg_max_n (0 .. 128), the
+   * blocked kernels in a workspace above; f64_strip16_max_n (0 .. 64) is accepted and has
+   * no effect */
   int32_t f64_reg_max_n;
   int32_t f64_strip16_max_n;
   /* blocked float32 Parlett-Reid: the batch runs as two halves, each launch holding one
@@ -327,8 +327,8 @@ int fx_slogpf_parts_f32(const float* a, int64_t batch, int32_t n, int32_t skew_s
  * The reference takes float64 through the same API (`_prep`, src/fermix/api.py:24-31,
  * with 64-bit fields, src/fermix/_field.py:20-120 and :265-275). These entry points are
  * the float64 counterparts of the ones above, with the same argument meaning, outputs
- * in float64 and 0 <= n <= 8192. For n <= fx_tune.f64_reg_max_n (128) one workgroup per
- * matrix holds it in registers: an LU / Gauss-Jordan with partial pivoting
+ * in float64 and 0 <= n <= 8192. For n <= fx_tune.f64_reg_max_n (128) one workgroup (a
+ * wave for n <= 32) per matrix holds it in LDS: an LU / Gauss-Jordan with partial pivoting
  * (`_slogdet_generic`, `_lu_parts_generic`, src/fermix/_fallback.py:36-97) and
  * Parlett-Reid (`_slogpf_generic`, :266-300), no workspace. Above, slogdet / det and the
  * inverses run a blocked LU (32-column panels, the trailing updates on the fp64 MFMA) and
@@ -380,16 +380,15 @@ int fx_slogpf_parts_f64(const double* a, int64_t batch, int32_t n, int32_t skew_
  * of largest |re| + |im| (LAPACK's cabs1, the reference's `abs1`), sign = parity *
  * prod(d / |d|), logabs = sum log|d|, an exactly zero pivot gives sign 0 and logabs -inf;
  * inv_t = A^-T without conjugation (the holomorphic derivative of log det, as in
- * `_lu_parts_generic`, :63-97). 0 <= n <= 8192. Up to n = 64 one workgroup per matrix,
- * the matrix in LDS when it fits (else one copy per member in the workspace; twice that
- * with the inverse); above, the blocked kernels of the float64 path on the complex field
+ * `_lu_parts_generic`, :63-97). 0 <= n <= 8192. Up to n = 128 (the LU of complex128:
+ * 96) one launch with the matrix in LDS; above, the blocked kernels of the float64 path on the complex field
  * (32-column LU panels, 16-pair Parlett-Reid panels, the trailing updates as four real
  * MFMA products per complex one). The complex64 entry points take prec:
  * FX_PREC_BF16X3 (the fp32-accuracy mode, the Python API's default as for float32) forms
  * those products on the fp64 MFMA with the operands widened to double; FX_PREC_IEEE as
  * four fp32 MFMA products (the reference's complex64 fp32-rate products, _field.py:173-190;
  * the fp32 MFMA's rate and rounding). Any other value: FX_ERR_INVALID_ARGUMENT. Up to
- * n = 64 (no blocked products) both give the same bits. complex128 has no prec (IEEE
+ * n = 128 (no blocked kernels; the products on the fp64 MFMA) both give the same bits. complex128 has no prec (IEEE
  * fp64). */
 size_t fx_slogdet_c64_workspace(int64_t batch, int32_t n);
 int fx_slogdet_c64(const float* a, int64_t batch, int32_t n, float* sign, float* logabs, int32_t prec,
@@ -428,8 +427,8 @@ int fx_slogpf_c128(const double* a, int64_t batch, int32_t n, int32_t skew_symme
  * inverse of the replaced factorisation, a second exact zero pivot lifted to +1 and -1
  * (two inverses for those members); above n = 64 only the members with pf = 0 or a
  * numerically singular S (the forward's pair pivots spanning more than 2^8 in modulus for
- * complex64, 2^18 for complex128) take that route, the others pf(S) times S^-1 from the
- * blocked LU solves; sign / logabs stay those of the plain forward. */
+ * complex64, 2^18 for complex128) take that route, the others pf(S) times S^-1 from an
+ * LU of S; sign / logabs stay those of the plain forward. */
 size_t fx_slogpf_parts_c64_workspace(int64_t batch, int32_t n);
 int fx_slogpf_parts_c64(const float* a, int64_t batch, int32_t n, int32_t skew_symmetrize, int32_t adjugate,
                         float* sign, float* logabs, float* g, int32_t prec, void* workspace, size_t workspace_bytes,
