@@ -331,7 +331,7 @@ int inv_padded(int N) {
 }
 
 size_t lu_inverse_workspace(int64_t batch, int N, bool need_copy) {
-  if (N <= SMALL_INV_MAXN) return ((size_t)batch * 4 + 255) / 256 * 256;  // nominal: nothing is kept there
+  if (N <= SMALL_INV_MAXN) return ((size_t)batch * 32 + 255) / 256 * 256;  // nominal, left unused
   const int Ninv = inv_padded(N);
   const int nt = (N + 63) / 64;  // 64x64 tiles of the Z product
   size_t bytes = 0;

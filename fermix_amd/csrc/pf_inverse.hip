@@ -269,7 +269,7 @@ __global__ __launch_bounds__(256) void pf_zero_bad_kernel(const int* __restrict_
 }
 
 size_t pf_inverse_workspace(int64_t batch, int N) {
-  if (N <= SMALL_INV_MAXN) return ((size_t)batch * 4 + 255) / 256 * 256;  // nominal: nothing is kept there
+  if (N <= SMALL_INV_MAXN) return ((size_t)batch * 32 + 255) / 256 * 256;  // nominal, left unused
   const int Ninv = inv_padded(N);
   size_t bytes = 0;
   auto add = [&](size_t x) { bytes += (x + 255) / 256 * 256; };
