@@ -69,10 +69,16 @@ def _on_device(a):
 def _flat(a):
     batch = a.shape[:-2]
     n = a.shape[-1]
+    if a.dim() == 3:
+        return a.contiguous(), batch, n
     B = 1
     for d in batch:
         B *= int(d)
     return a.reshape((B, n, n)).contiguous(), batch, n
+
+
+def _shaped(x, batch):
+    return x if len(batch) == 1 else x.reshape(batch)
 
 
 def _lu_opts(a, prec, unroll_steps, block):
@@ -101,7 +107,7 @@ def slogdet(a, *, prec=None, unroll_steps=None, block=None):
     _on_device(a)
     A, batch, n = _flat(a)
     sign, logabs = _diff.slogdet(A, x3)
-    return sign.reshape(batch), logabs.reshape(batch)
+    return _shaped(sign, batch), _shaped(logabs, batch)
 
 
 def slogpf(a, *, prec=None, skew_symmetrize=True, upd_warps=None):
@@ -119,9 +125,9 @@ def slogpf(a, *, prec=None, skew_symmetrize=True, upd_warps=None):
     A, batch, n = _flat(a)
     if n % 2 == 1:
         sign, logabs = _diff.odd_slogpf(A)
-        return sign.reshape(batch), logabs.reshape(batch)
+        return _shaped(sign, batch), _shaped(logabs, batch)
     sign, logabs = _diff.slogpf(A, bool(skew_symmetrize), x3)
-    return sign.reshape(batch), logabs.reshape(batch)
+    return _shaped(sign, batch), _shaped(logabs, batch)
 
 
 def det(a, *, prec=None, unroll_steps=None, block=None):
@@ -131,7 +137,7 @@ def det(a, *, prec=None, unroll_steps=None, block=None):
     x3 = _lu_opts(a, prec, unroll_steps, block)
     _on_device(a)
     A, batch, n = _flat(a)
-    return _diff.det(A, x3).reshape(batch)
+    return _shaped(_diff.det(A, x3), batch)
 
 
 def pf(a, *, prec=None, skew_symmetrize=True, upd_warps=None):
@@ -143,8 +149,8 @@ def pf(a, *, prec=None, skew_symmetrize=True, upd_warps=None):
     _on_device(a)
     A, batch, n = _flat(a)
     if n % 2 == 1:
-        return _diff.odd_pf(A).reshape(batch)
-    return _diff.pf(A, bool(skew_symmetrize), x3).reshape(batch)
+        return _shaped(_diff.odd_pf(A), batch)
+    return _shaped(_diff.pf(A, bool(skew_symmetrize), x3), batch)
 
 
 __all__ = [
