@@ -550,10 +550,11 @@ int lu_values(const F* a, int n, int64_t batch, F* sign, typename Fd<F>::R* loga
 }
 template <class F>
 int lu_inverse(const F* a, int n, int skew, int64_t batch, F* sign, typename Fd<F>::R* logabs, const F* gate,
-               const F* ssign, const typename Fd<F>::R* slog, F* out, int out_t, void* ws, size_t wsb, hipStream_t s) {
+               const F* ssign, const typename Fd<F>::R* slog, F* out, int out_t, void* ws, size_t wsb, hipStream_t s,
+               SideStream* side = nullptr) {
   if constexpr (!std::is_same<F, float>::value)
     if (lds_lu<F>(n)) return fsmall_lu<F>(a, n, skew, batch, sign, logabs, gate, ssign, slog, out, out_t, s);
-  return blk_lu_inverse<F>(a, n, skew, batch, sign, logabs, gate, ssign, slog, out, out_t, ws, wsb, s);
+  return blk_lu_inverse<F>(a, n, skew, batch, sign, logabs, gate, ssign, slog, out, out_t, ws, wsb, s, side);
 }
 template <class F>
 int pr_values(const F* a, int n, int skew, int64_t batch, F* sign, typename Fd<F>::R* logabs, void* ws, size_t wsb,
@@ -765,7 +766,10 @@ int blk_pf_parts(const F* A, int64_t batch, int n, int skew, int adjugate, F* si
   char* base = (char*)ws;
   double* spread = (double*)(base + pr + body);
   F* gz = (F*)(base + pr + body + align_up((size_t)batch * sizeof(double)));
-  int st = pr_values<F>(A, n, skew, batch, sign, logabs, base, pr, s, spread);
+  SideStream side(s, !adjugate && !lds_lu<F>(n) && pf_parts_overlap(batch, n));
+  int st = side.ok() ? side.fork() : FX_OK;
+  if (st != FX_OK) return st;
+  st = pr_values<F>(A, n, skew, batch, sign, logabs, base, pr, side.side(), spread);
   if (st != FX_OK) return st;
   if (adjugate && (n & 1)) return cx_zero<F>(g, batch * (int64_t)n * n, s);
   F* gsign = (F*)(base + pr + lw);
@@ -777,7 +781,7 @@ int blk_pf_parts(const F* A, int64_t batch, int n, int skew, int adjugate, F* si
     gate = gz;
   }
   st = lu_inverse<F>(A, n, skew, batch, gsign, glog, gate, adjugate ? sign : nullptr, adjugate ? logabs : nullptr, g, 0,
-                     base + pr, lw, s);
+                     base + pr, lw, s, &side);
   if (st != FX_OK || !adjugate) return st;
   return pf_adjugate<F>(A, batch, n, skew, g, base + pr, body, s, gate);
 }

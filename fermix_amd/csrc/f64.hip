@@ -218,7 +218,9 @@ int fx_slogpf_parts_f64(const double* a, int64_t batch, int32_t n, int32_t skew_
   const size_t pr = align_up_256(fx_slogpf_f64_workspace(batch, n));
   char* base = (char*)workspace;
   double* spread = lu64_path(n) ? (double*)(base + need - align_up_256((size_t)batch * sizeof(double))) : nullptr;
-  st = lu64_path(n) ? launch_pr64_blocked(a, n, skew_symmetrize != 0, batch, sign, logabs, base, pr, s, spread)
+  SideStream side(s, !adjugate && lu64_path(n) && pf_parts_overlap(batch, n));
+  if (side.ok() && (st = side.fork()) != FX_OK) return st;
+  st = lu64_path(n) ? launch_pr64_blocked(a, n, skew_symmetrize != 0, batch, sign, logabs, base, pr, side.side(), spread)
                     : fsmall_pr<double>(a, n, skew_symmetrize != 0, batch, sign, logabs, s);
   if (st != FX_OK || n == 0) return st;
   // the Pfaffian adjugate (cplx.hip): the LU route, or the pivot-replaced Parlett-Reid
@@ -232,7 +234,7 @@ int fx_slogpf_parts_f64(const double* a, int64_t batch, int32_t n, int32_t skew_
     const size_t lw = align_up_256(lu64_inverse_workspace(batch, n));
     double* gsign = (double*)(base + pr + lw);
     return launch_lu64_inverse(a, n, skew_symmetrize != 0, batch, gsign, gsign + batch, sign, nullptr, nullptr, g, 0,
-                               base + pr, lw, s);
+                               base + pr, lw, s, &side);
   }
   double* gsign = (double*)(base + pr);
   return fsmall_lu<double>(a, n, skew_symmetrize != 0, batch, gsign, gsign + batch, sign, nullptr, nullptr, g, 0, s);

@@ -200,6 +200,13 @@ int launch_gemm(const GemmDesc& d, int64_t batch, int nb2, hipStream_t s);
 // determinant with det), zero for singular members
 int launch_lu64_small(const double* a, int n, int64_t batch, double* sign, double* logabs, double* out, bool det,
                       hipStream_t s);
+// Whether a parts run's Parlett-Reid goes beside its LU on the side stream: both are chains of
+// panels on one workgroup per matrix that leave most of a CU idle. slogpf + S^-1, alone ->
+// beside, us: float64 B = 48, n = 302 1950 -> 1395, B = 200, n = 302 3286 -> 2846, B = 512, n =
+// 200 2919 -> 2794, B = 1000, n = 140 2644 -> 2576; the gain fades with the batch, so not above
+// 1024. Not above n = 512, where panels span several cooperatively launched workgroups that
+// must all be resident.
+inline bool pf_parts_overlap(int64_t batch, int n) { return n <= 512 && batch <= 1024; }
 // float64 blocked LU (sign, logabs) for the orders above the register kernels (lu64_impl.inc)
 size_t lu64_workspace(int64_t batch, int n);
 int launch_lu64(const double* A, int n, int64_t batch, double* sign, double* logabs, void* ws, size_t ws_bytes,
@@ -211,7 +218,7 @@ int launch_lu64(const double* A, int n, int64_t batch, double* sign, double* log
 size_t lu64_inverse_workspace(int64_t batch, int n);
 int launch_lu64_inverse(const double* A, int n, int skew, int64_t batch, double* sign, double* logabs,
                         const double* gate, const double* ssign, const double* slog, double* out, int out_t,
-                        void* ws, size_t ws_bytes, hipStream_t s);
+                        void* ws, size_t ws_bytes, hipStream_t s, SideStream* side = nullptr);
 // float64 Parlett-Reid sign / logabs for n above the register kernels (lu64_impl.inc): 16 pair
 // steps per panel, the trailing update on the fp64 MFMA
 size_t pr64_workspace(int64_t batch, int n);

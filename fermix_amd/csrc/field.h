@@ -141,7 +141,7 @@ __device__ __forceinline__ float half_diff(float v, float u) { return (v - u) * 
 // The blocked LU, its solves and the blocked Parlett-Reid for F = double, cx<float>,
 // cx<double> (lu64_impl.inc): sign / logabs, and out = A^-T / A^-1 (times ssign exp(slog) when
 // ssign is given, zero where gate -- default: the factorisation's own sign -- is 0 or the
-// result is not finite); 0 < n <= blk_max_n<F>(), every buffer of the batch.
+// result is not finite; side: joined before gate, ssign and slog are read); 0 < n <= blk_max_n<F>(), every buffer of the batch.
 template <class F>
 size_t blk_lu_workspace(int64_t batch, int n);
 template <class F>
@@ -152,7 +152,7 @@ size_t blk_lu_inverse_workspace(int64_t batch, int n);
 template <class F>
 int blk_lu_inverse(const F* A, int n, int skew, int64_t batch, F* sign, typename Fd<F>::R* logabs, const F* gate,
                    const F* ssign, const typename Fd<F>::R* slog, F* out, int out_t, void* ws, size_t ws_bytes,
-                   hipStream_t s);
+                   hipStream_t s, SideStream* side = nullptr);
 template <class F>
 size_t blk_pr_workspace(int64_t batch, int n);
 template <class F>
