@@ -312,7 +312,7 @@ __device__ __forceinline__ void load_tile(float* As, const float* __restrict__ g
       for (int u = 0; u < CH; ++u) {
         const int e = base + tid + NT * u;
         const int r = e / N, c = e % N;
-        v[u] = (e < N * N && r < n && c < n) ? g[r * n + c] : 0.0f;
+        v[u] = g[min(r, n - 1) * n + min(c, n - 1)];  // outside the matrix: its edge, unused
       }
 #pragma unroll
       for (int u = 0; u < CH; ++u) {

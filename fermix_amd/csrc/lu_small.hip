@@ -221,7 +221,7 @@ __global__ __launch_bounds__(256) void lu_small_kernel(const float* __restrict__
                                                        float* __restrict__ lu_out,
                                                        int* __restrict__ perm_out) {
   constexpr int LDA = LuSmall<N>::LDA, NP = LuSmall<N>::NP;
-  __shared__ float As[N * LDA];
+  __shared__ __align__(16) float As[N * LDA];
   __shared__ int srcs[2][N];
   __shared__ float Xs[2][256];
   __shared__ int perm[N];
@@ -266,9 +266,9 @@ __global__ __launch_bounds__(256) void lu_small_kernel(const float* __restrict__
   }
   if (FACT) {
     float* Lb = lu_out + b * (int64_t)N * N;
-    for (int e = tid; e < N * N; e += 256) {
-      const int r = e / N, c = e - r * N;
-      Lb[e] = As[r * LDA + c];
+    for (int e = tid; e < N * N / 4; e += 256) {
+      const int r = e / (N / 4), c = 4 * (e % (N / 4));
+      *reinterpret_cast<v4f*>(Lb + r * N + c) = *reinterpret_cast<const v4f*>(As + r * LDA + c);
     }
     for (int r = tid; r < N; r += 256) perm_out[b * N + r] = perm[r];
   }
@@ -291,6 +291,8 @@ __global__ __launch_bounds__(256) void lu_small_kernel(const float* __restrict__
 // Products whose right operand sits in accumulator layout (lane (g, c) holding rows
 // 4g + v of a 16 x 16 tile) take it as it stands, one MFMA per v over the K indices
 // {4g + v}, with the left operand read from LDS in that order.
+// The ragged orders read 16-byte (n % 4 == 0) or batched 4-byte pieces without branches: B = 4096, n =
+// 100 243 -> 212 us, n = 127 281 -> 234 (n = 128 225).
 // Four workgroups per CU: at most 128 registers per lane (the compiler fits 111 without
 // scratch at N = 128) and 40,448 bytes of LDS.
 template <int N, int H, bool FACT>
@@ -306,7 +308,7 @@ __global__ __launch_bounds__(256, 4) void lu_split_kernel(const float* __restric
   constexpr int NPV = (N + 63) / 64;
   static_assert(H % 16 == 0 && NS % 16 == 0 && NPS <= 4 && NS <= H, "split shape");
   static_assert(NS * LDS_ <= H * LDH, "S must not reach the rows of L21");
-  __shared__ float As[N * LDH];        // N x H left block, later the NS x NS complement
+  __shared__ __align__(16) float As[N * LDH];  // N x H left block, later the NS x NS complement
   __shared__ int srcs[2][N];
   __shared__ float Xall[NPH][256];     // X = L_ss^-1 of every left panel (phase 2)
   __shared__ int perm[N];
@@ -335,10 +337,38 @@ __global__ __launch_bounds__(256, 4) void lu_split_kernel(const float* __restric
         d[3] = v[i].w;
       }
     }
+  } else if ((n & 3) == 0) {
+    // 16-byte pieces; those outside the matrix are read at its last row or columns (no
+    // branch) and replaced by the identity
+    constexpr int NV = N * H / 4, PER = (NV + 255) / 256;
+    v4f v[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int e = min(tid + 256 * i, NV - 1), r = e / (H / 4), c = 4 * (e % (H / 4));
+      v[i] = *reinterpret_cast<const v4f*>(Ab + min(r, n - 1) * n + min(c, n - 4));
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int e = min(tid + 256 * i, NV - 1), r = e / (H / 4), c = 4 * (e % (H / 4));
+      const bool in = r < n && c < n;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[i][u] = in ? v[i][u] : (r == c + u ? 1.0f : 0.0f);
+      *reinterpret_cast<v4f*>(As + r * LDH + c) = v[i];
+    }
   } else {
-    for (int e = tid; e < N * H; e += 256) {
-      const int r = e / H, c = e % H;
-      As[r * LDH + c] = (r < n && c < n) ? Ab[r * n + c] : (r == c ? 1.0f : 0.0f);
+    constexpr int CH = 16;
+    for (int base = 0; base < N * H; base += 256 * CH) {
+      float v[CH];
+#pragma unroll
+      for (int u = 0; u < CH; ++u) {
+        const int e = base + tid + 256 * u, r = e / H, c = e % H;
+        v[u] = Ab[min(r, n - 1) * n + min(c, n - 1)];
+      }
+#pragma unroll
+      for (int u = 0; u < CH; ++u) {
+        const int e = base + tid + 256 * u, r = e / H, c = e % H;
+        if (N * H % (256 * CH) == 0 || e < N * H) As[r * LDH + c] = (r < n && c < n) ? v[u] : (r == c ? 1.0f : 0.0f);
+      }
     }
   }
   for (int r = tid; r < N; r += 256) perm[r] = r;
@@ -367,7 +397,10 @@ __global__ __launch_bounds__(256, 4) void lu_split_kernel(const float* __restric
 
   if (FACT) {
     // rows 0 .. H-1 of the left block are final: L11 \ U11
-    for (int e = tid; e < H * H; e += 256) Lb[(e / H) * N + e % H] = As[(e / H) * LDH + e % H];
+    for (int e = tid; e < H * H / 4; e += 256) {
+      const int r = e / (H / 4), c = 4 * (e % (H / 4));
+      *reinterpret_cast<v4f*>(Lb + r * N + c) = *reinterpret_cast<const v4f*>(As + r * LDH + c);
+    }
   }
 
   // phase 2: wave w forms columns H + 16w .. H + 16w + 15 of S
@@ -377,7 +410,8 @@ __global__ __launch_bounds__(256, 4) void lu_split_kernel(const float* __restric
     const int c = H + 16 * wave + li;
     auto elem = [&](int p) {
       const int r = perm[p];
-      return (r < n && c < n) ? Ab[__umul24(r, n) + c] : (r == c ? 1.0f : 0.0f);
+      const float x = Ab[__umul24(min(r, n - 1), n) + min(c, n - 1)];
+      return (r < n && c < n) ? x : (r == c ? 1.0f : 0.0f);
     };
     v4f ap[NPH];
 #pragma unroll
@@ -463,9 +497,10 @@ __global__ __launch_bounds__(256, 4) void lu_split_kernel(const float* __restric
   }
   if (FACT) {
     // rows H .. N-1: L21 and the packed LU of S
-    for (int e = tid; e < NS * N; e += 256) {
-      const int r = e / N, c = e % N;
-      Lb[(H + r) * N + c] = c < H ? L21[r * LDH + c] : As[r * LDS_ + c - H];
+    for (int e = tid; e < NS * N / 4; e += 256) {
+      const int r = e / (N / 4), c = 4 * (e % (N / 4));
+      *reinterpret_cast<v4f*>(Lb + (H + r) * N + c) =
+          *reinterpret_cast<const v4f*>(c < H ? L21 + r * LDH + c : As + r * LDS_ + c - H);
     }
     for (int r = tid; r < N; r += 256) perm_out[b * N + r] = perm[r];
   }

@@ -337,57 +337,74 @@ __device__ __forceinline__ void pf_load_full(float* T, const float* __restrict__
   }
 }
 
-// Load the matrix (row-major n x n, n even) into T, padded with [[0,1],[-1,0]] blocks;
-// with skew, T holds (A - A^T) / 2 formed as A[p][q] / 2 - A[q][p] / 2 (halving is exact).
-template <int N>
+// The same for an even n < N, rows of 8-byte (V = 2) or, with n a multiple of 4, 16-byte
+// (V = 4) aligned pieces: loads outside the matrix go to its last row or columns instead (they
+// need no branch) and their entries to the padding [[0,1],[-1,0]]. In place of element-wise
+// loads with a second pass that subtracted the transposed entries in LDS behind a barrier:
+// B = 4096, n = 98 213 -> 135 us, n = 114 255 -> 162, n = 66 95 -> 70 (as n = N).
+template <int N, int V>
+__device__ __forceinline__ void pf_load_pad(float* T, const float* __restrict__ g, int n, int skew, int tid) {
+  constexpr int NB4 = N / 4;
+  constexpr int NPAIR = NB4 * (NB4 + 1) / 2;
+  constexpr int ITER = (NPAIR + 255) / 256;
+  float lo[ITER][4][4], up[ITER][4][4];
+  int bi[ITER], bj[ITER];
+  auto block = [&](int r0, int c0, float (&x)[4][4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float* row = g + __umul24(min(r0 + i, n - 1), n);
+      if constexpr (V == 4) {
+        const float4 v = *reinterpret_cast<const float4*>(row + min(c0, n - 4));
+        x[i][0] = v.x;
+        x[i][1] = v.y;
+        x[i][2] = v.z;
+        x[i][3] = v.w;
+      } else {
+        const float2 v = *reinterpret_cast<const float2*>(row + min(c0, n - 2));
+        const float2 w = *reinterpret_cast<const float2*>(row + min(c0 + 2, n - 2));
+        x[i][0] = v.x;
+        x[i][1] = v.y;
+        x[i][2] = w.x;
+        x[i][3] = w.y;
+      }
+    }
+  };
+#pragma unroll
+  for (int it = 0; it < ITER; ++it) {
+    const int t = min(tid + 256 * it, NPAIR - 1);
+    const int f = t / (NB4 + 1), x = t - f * (NB4 + 1);
+    bi[it] = x <= f ? f : NB4 - 1 - f;
+    bj[it] = x <= f ? x : x - f - 1;
+    block(4 * bi[it], 4 * bj[it], lo[it]);
+    if (skew) block(4 * bj[it], 4 * bi[it], up[it]);
+  }
+#pragma unroll
+  for (int it = 0; it < ITER; ++it) {
+    const int p0 = 4 * bi[it], q0 = 4 * bj[it];
+    if (NPAIR % 256 == 0 || tid + 256 * it < NPAIR) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int p = p0 + i;
+        float* d = T + tri_row(p) + q0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          float v = skew ? fmaf(-up[it][j][i], 0.5f, lo[it][i][j] * 0.5f) : lo[it][i][j];
+          if (p >= n) v = (i & 1) && q0 + j == p - 1 ? -1.0f : 0.0f;
+          if (i > j || p0 != q0) d[j] = v;
+        }
+      }
+    }
+  }
+}
+
+// Load the matrix (row-major n x n, n even) into T, padded with [[0,1],[-1,0]] blocks (PAD;
+// n == N without); with skew, T holds (A - A^T) / 2 formed as A[p][q] / 2 - A[q][p] / 2
+// (halving is exact).
+template <int N, bool PAD>
 __device__ __forceinline__ void pf_load(float* T, const float* __restrict__ g, int n, int skew, int tid) {
-  const float h = skew ? 0.5f : 1.0f;
-  if (n == N) {
-    pf_load_full<N>(T, g, skew, tid);
-    return;
-  }
-  {
-    // lower triangle (every entry written once), then the upper halves subtracted
-    constexpr int CH = 8;
-    for (int base = 0; base < N * N; base += 256 * CH) {
-      float v[CH];
-#pragma unroll
-      for (int u = 0; u < CH; ++u) {
-        const int e = base + tid + 256 * u;
-        const int r = e / N, c = e % N;
-        v[u] = (e < N * N && r < n && c < r) ? g[r * n + c] : 0.0f;
-      }
-#pragma unroll
-      for (int u = 0; u < CH; ++u) {
-        const int e = base + tid + 256 * u;
-        const int r = e / N, c = e % N;
-        // padding: M[2m+1][2m] = -1 below the n x n block
-        if (e < N * N && c < r)
-          T[tri_row(r) + c] = (r < n) ? v[u] * h : ((c == r - 1 && (r & 1)) ? -1.0f : 0.0f);
-      }
-    }
-    if (skew) {
-      __syncthreads();
-      for (int base = 0; base < N * N; base += 256 * CH) {
-        float v[CH];
-#pragma unroll
-        for (int u = 0; u < CH; ++u) {
-          const int e = base + tid + 256 * u;
-          const int r = e / N, c = e % N;
-          v[u] = (e < N * N && c < n && r < c) ? g[r * n + c] : 0.0f;
-        }
-#pragma unroll
-        for (int u = 0; u < CH; ++u) {
-          const int e = base + tid + 256 * u;
-          const int r = e / N, c = e % N;
-          if (e < N * N && c < n && r < c) {
-            float* d = T + tri_row(c) + r;
-            *d = *d - v[u] * 0.5f;
-          }
-        }
-      }
-    }
-  }
+  if constexpr (!PAD) pf_load_full<N>(T, g, skew, tid);
+  else if ((n & 3) == 0) pf_load_pad<N, 4>(T, g, n, skew, tid);
+  else pf_load_pad<N, 2>(T, g, n, skew, tid);
 }
 
 // Trailing update of one block: M'' = M + G J G^T (J = diag of [[0,1],[-1,0]]) over the
@@ -489,7 +506,9 @@ __device__ __forceinline__ void pf_update(float* T, const float* Gs, const unsig
   }
 }
 
-template <int N, bool FACT>
+// PAD: n < N. A kernel of its own: in one kernel the padded loads' registers cost the n == N
+// call 1 % (B = 4096, n = 128 165.7 -> 167.3 us).
+template <int N, bool FACT, bool PAD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void pf_small_kernel(const float* __restrict__ A, int n, int skew,
                                                        float* __restrict__ sign_out,
                                                        float* __restrict__ logabs_out,
@@ -505,7 +524,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
   __shared__ unsigned char orig[FACT ? N : 1];
   const int64_t b = blockIdx.x;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  pf_load<N>(T, A + b * (int64_t)n * n, n, skew, tid);
+  pf_load<N, PAD>(T, A + b * (int64_t)n * n, n, skew, tid);
   if (FACT)
     for (int r = tid; r < N; r += 256) orig[r] = (unsigned char)r;
   __syncthreads();
@@ -549,8 +568,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
 template <int N, bool FACT>
 static int launch_n(const float* A, int n, int skew, int64_t batch, float* sign, float* logabs,
                     float* gbuf, float* d, int* perm, hipStream_t s) {
-  hipLaunchKernelGGL((pf_small_kernel<N, FACT>), dim3((unsigned)batch), dim3(256), 0, s, A, n, skew,
-                     sign, logabs, gbuf, d, perm);
+  if (n == N)
+    hipLaunchKernelGGL((pf_small_kernel<N, FACT, false>), dim3((unsigned)batch), dim3(256), 0, s, A, n, skew,
+                       sign, logabs, gbuf, d, perm);
+  else
+    hipLaunchKernelGGL((pf_small_kernel<N, FACT, true>), dim3((unsigned)batch), dim3(256), 0, s, A, n, skew,
+                       sign, logabs, gbuf, d, perm);
   return hipGetLastError() == hipSuccess ? FX_OK : FX_ERR_LAUNCH;
 }
 

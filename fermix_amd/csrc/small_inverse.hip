@@ -352,8 +352,14 @@ __global__ __launch_bounds__(SmallInv<NB>::NT, SmallInv<NB>::WPE) void lu_inv_sm
         for (int i = 0; i < NB; ++i) *reinterpret_cast<v4f*>(T + row[c] * LD + 16 * i + 4 * g) = bad ? zero : sc * opaque4(z[c][i]);
       }
     mat_sync<NW>();
-    for (int r = wave; r < n; r += NW)
-      for (int e = lane; e < n; e += 64) ob[(int64_t)r * n + e] = T[r * LD + e];
+    if ((n & 1) == 0) {
+      for (int r = wave; r < n; r += NW)
+        if (2 * lane < n)
+          *reinterpret_cast<float2*>(ob + (int64_t)r * n + 2 * lane) = *reinterpret_cast<const float2*>(T + r * LD + 2 * lane);
+    } else {
+      for (int r = wave; r < n; r += NW)
+        for (int e = lane; e < n; e += 64) ob[(int64_t)r * n + e] = T[r * LD + e];
+    }
   }
 }
 
@@ -581,12 +587,19 @@ __global__ __launch_bounds__(SmallInv<NB>::NT, SmallInv<NB>::WPE) void pf_inv_sm
         v4f* o = reinterpret_cast<v4f*>(ob + 4 * e);
         *o = pass ? *o + sc * val : sc * val;
       }
-    } else {
-      for (int e = tid; e < n * n; e += TM) {
-        const int x = e / n, y = e - x * n;
-        const float val = -(a1 * T[x * LD + y] + a2 * wedge(ws[m][x], vs[m][y], vs[m][x], ws[m][y]));
-        nf = nf || !isfinite(val);
-        ob[e] = pass ? ob[e] + sc * val : sc * val;
+    } else {  // n is even: 8-byte rows
+      const int n2 = n >> 1;
+      for (int e = tid; e < n * n2; e += TM) {
+        const int x = e / n2, y = 2 * (e - x * n2);
+        const float wx = ws[m][x], vx = vs[m][x];
+        const float2 rr = *reinterpret_cast<const float2*>(T + x * LD + y);
+        const float2 wy = *reinterpret_cast<const float2*>(&ws[m][y]), vy = *reinterpret_cast<const float2*>(&vs[m][y]);
+        const float v0 = -(a1 * rr.x + a2 * wedge(wx, vy.x, vx, wy.x));
+        const float v1 = -(a1 * rr.y + a2 * wedge(wx, vy.y, vx, wy.y));
+        nf = nf || !isfinite(v0) || !isfinite(v1);
+        float2* o = reinterpret_cast<float2*>(ob + 2 * e);
+        const float2 old = pass ? *o : make_float2(0.0f, 0.0f);
+        *o = make_float2(old.x + sc * v0, old.y + sc * v1);
       }
     }
     // inverse mode: a member with d_K = 0 or a non-finite value is cleared (each thread
@@ -595,7 +608,7 @@ __global__ __launch_bounds__(SmallInv<NB>::NT, SmallInv<NB>::WPE) void pf_inv_sm
       if ((n & 3) == 0) {
         for (int e = tid; e < n * (n >> 2); e += TM) *reinterpret_cast<v4f*>(ob + 4 * e) = zero;
       } else {
-        for (int e = tid; e < n * n; e += TM) ob[e] = 0.0f;
+        for (int e = tid; e < n * (n >> 1); e += TM) *reinterpret_cast<float2*>(ob + 2 * e) = make_float2(0.0f, 0.0f);
       }
     }
   }
