@@ -324,6 +324,20 @@ __device__ __forceinline__ void load_tile(float* As, const float* __restrict__ g
   }
 }
 
+// The lowest wave w < NW (a power of two, at most 16) whose key, held by the lanes w mod NW, is
+// the largest; wave-uniform. Three or four DPP steps, where a scan of the posts took a
+// dependent compare and two selects per wave.
+template <int NW>
+__device__ __forceinline__ int best_wave(unsigned k) {
+  if constexpr (NW == 1) return 0;
+  unsigned v = k;
+  v = max(v, dpp_u32<0xB1>(v));                          // quad_perm [1,0,3,2]
+  if constexpr (NW > 2) v = max(v, dpp_u32<0x4E>(v));    // quad_perm [2,3,0,1]
+  if constexpr (NW > 4) v = max(v, dpp_u32<0x141>(v));   // row_half_mirror
+  if constexpr (NW > 8) v = max(v, dpp_u32<0x140>(v));   // row_mirror
+  return (int)__builtin_ctzll(__ballot(k == v));
+}
+
 // ---- 64-bit workgroup argmax (the float64 and complex kernels)
 
 // Order-preserving key of a pivot candidate: |x| bits plus one (0 = no candidate).

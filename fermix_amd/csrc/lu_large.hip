@@ -315,11 +315,14 @@ __global__ __launch_bounds__(NT) void lu_panel_reg_kernel(float* __restrict__ W,
                                                           int* __restrict__ g0,
                                                           const float* __restrict__ A0, int lmove) {
   constexpr int NW = NT / 64, PW = 64, NSUB = 4;
-  __shared__ Cand cand[2][NW];
+  // one post per wave: the keys side by side, each post's row, position and 16 entries
+  __shared__ __align__(16) float candv[2][NW][16];
+  __shared__ unsigned candk[2][NW];
+  __shared__ int2 candp[2][NW];
   __shared__ __align__(16) float Prow[16 * PW];  // pivot rows of the sub-panel, all columns
   __shared__ __align__(16) float Ubuf[16 * PW];
-  __shared__ float Xs[256];
-  __shared__ float L11s[256];
+  __shared__ __align__(16) float Xs[256];
+  __shared__ __align__(16) float L11s[256];
   const int64_t b = blockIdx.x;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int m = N - r0;
@@ -343,6 +346,7 @@ __global__ __launch_bounds__(NT) void lu_panel_reg_kernel(float* __restrict__ W,
     }
   }
   int nsw = 0;
+  float mypiv = 0.0f;  // the pivot of this row's column, once it is one
   static_for<0, NSUB>([&](auto spc) {
     constexpr int c0 = 16 * decltype(spc)::value;
     static_for<0, 16>([&](auto jc) {
@@ -351,34 +355,38 @@ __global__ __launch_bounds__(NT) void lu_panel_reg_kernel(float* __restrict__ W,
       const unsigned kb = cand_key(a[col], valid && pos >= col);
       const unsigned gk = wave_max_u32(kb);
       const int pl = first_lane(gk != 0u ? (kb == gk) : (lane == 0));
-      Cand& my = cand[j & 1][wave];
       if (lane == pl) {
-        my.key = gk;
-        my.row = tid;
-        my.pos = pos;
+        candk[j & 1][wave] = gk;
+        candp[j & 1][wave] = make_int2(tid, pos);
 #pragma unroll
-        for (int jj = 0; jj < 16; ++jj) my.v[jj] = a[c0 + jj];
+        for (int jj = 0; jj < 16; jj += 4)
+          *reinterpret_cast<float4*>(&candv[j & 1][wave][jj]) =
+              make_float4(a[c0 + jj], a[c0 + jj + 1], a[c0 + jj + 2], a[c0 + jj + 3]);
       }
       __syncthreads();
-      unsigned best = cand[j & 1][0].key;
-      int wb = 0;
-#pragma unroll
-      for (int w = 1; w < NW; ++w) {
-        const unsigned kw = cand[j & 1][w].key;
-        if (kw > best) { best = kw; wb = w; }
-      }
-      const Cand& win = cand[j & 1][wb];
+      // the lowest wave of the largest key: lane w reads wave w's, reduced within NW lanes
+      const int wb = best_wave<NW>(candk[j & 1][lane & (NW - 1)]);
+      const float* const win = candv[j & 1][wb];
       float u[16];
 #pragma unroll
-      for (int jj = 0; jj < 16; ++jj) u[jj] = win.v[jj];
-      const int pp = win.pos, prow = win.row;
-      if (tid < j) L11s[j * 16 + tid] = win.v[tid];
+      for (int jj = j & ~3; jj < 16; jj += 4) {
+        const float4 x = *reinterpret_cast<const float4*>(win + jj);
+        u[jj] = x.x;
+        u[jj + 1] = x.y;
+        u[jj + 2] = x.z;
+        u[jj + 3] = x.w;
+      }
+      const int2 wp_ = candp[j & 1][wb];
+      const int pp = wp_.y, prow = wp_.x;
+      const float pivv = u[j];
       if (valid && pos == col) pos = pp;
-      if (tid == prow) pos = col;
+      if (tid == prow) {
+        pos = col;
+        mypiv = pivv;
+      }
+      mypiv = opaque(mypiv);  // taken here: its selects must not sink to the end with their operands
       nsw += (pp != col) ? 1 : 0;
       pin(nsw);
-      const float pivv = u[j];
-      if (tid == 0) piv_out[b * N + r0 + col] = pivv;
       const float rcp = safe_rcp(pivv);
       if (valid && pos > col) {
         const float l = a[col] * rcp;
@@ -386,9 +394,16 @@ __global__ __launch_bounds__(NT) void lu_panel_reg_kernel(float* __restrict__ W,
         static_for<j + 1, 16>([&](auto cc) { a[c0 + cc.value] = fmaf(-l, u[cc.value], a[c0 + cc.value]); });
       }
     });
-    if constexpr (c0 + 16 < PW) {
-      // the sub-panel's pivot rows publish their remaining columns
-      if (valid && pos >= c0 && pos < c0 + 16) {
+    // the sub-panel's pivot rows publish their row of L11 and their remaining columns (here,
+    // once, rather than a row of L11 in every step: that read and store stood before the
+    // step's barrier). With the posts reduced by best_wave, B = 8, n = 900 slogdet 1418 -> 1205 us, B =
+    // 95, n = 354 464 -> 425, B = 1024, n = 512 2364 -> 2263
+    if (valid && pos >= c0 && pos < c0 + 16) {
+      float* lr = L11s + (pos - c0) * 16;
+#pragma unroll
+      for (int c = 0; c < 16; c += 4)
+        *reinterpret_cast<float4*>(lr + c) = make_float4(a[c0 + c], a[c0 + c + 1], a[c0 + c + 2], a[c0 + c + 3]);
+      if constexpr (c0 + 16 < PW) {
         float* pr = Prow + (pos - c0) * PW;
 #pragma unroll
         for (int c = c0 + 16; c < PW; c += 4) *reinterpret_cast<float4*>(pr + c) = make_float4(a[c], a[c + 1], a[c + 2], a[c + 3]);
@@ -417,8 +432,21 @@ __global__ __launch_bounds__(NT) void lu_panel_reg_kernel(float* __restrict__ W,
       // U = X * Prow[:, c0+16 ..] (X unit lower: terms t <= k)
       for (int e = tid; e < 16 * NC; e += NT) {
         const int k = e / NC, c = c0 + 16 + e % NC;
+        // terms t < k in order, every operand read up front (a loop to k waited on each)
+        float xr[16], pr[16];
+#pragma unroll
+        for (int t = 0; t < 16; t += 4) {
+          const float4 v = *reinterpret_cast<const float4*>(Xs + k * 16 + t);
+          xr[t] = v.x;
+          xr[t + 1] = v.y;
+          xr[t + 2] = v.z;
+          xr[t + 3] = v.w;
+        }
+#pragma unroll
+        for (int t = 0; t < 15; ++t) pr[t] = Prow[t * PW + c];
         float s = Prow[k * PW + c];
-        for (int t = 0; t < k; ++t) s = fmaf(Xs[k * 16 + t], Prow[t * PW + c], s);
+#pragma unroll
+        for (int t = 0; t < 15; ++t) s = t < k ? fmaf(xr[t], pr[t], s) : s;
         Ubuf[k * PW + c] = s;
       }
       __syncthreads();
@@ -457,6 +485,7 @@ __global__ __launch_bounds__(NT) void lu_panel_reg_kernel(float* __restrict__ W,
 #pragma unroll
     for (int q = 0; q < PW / 4; ++q) wp[q] = make_float4(a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]);
     src_out[b * N + r0 + pos] = r0 + tid;
+    if (pos < PW) piv_out[b * N + r0 + pos] = mypiv;
   }
   if (lmove) {
     // the previous block's 64 L columns (left of the panel) follow the rows that moved:

@@ -55,9 +55,9 @@ static int pf_block_width(int N, int r0) {
 }
 
 struct PfCand {
-  unsigned key;
   int row;
   int pos;
+  int pad;
   float xv;  // x at the candidate row (d = -x[p])
   float g[PFB_L];
 };
@@ -169,6 +169,7 @@ __device__ __forceinline__ void pf_panel_body(const float* __restrict__ M, int N
   static_assert(PB % CW == 0 && PB / CW <= 2, "a block spans one or two chunks");
   __shared__ __align__(16) PfRowA rowa;
   __shared__ __align__(16) PfCand cand[2][NW];
+  __shared__ unsigned candk[2][NW];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int m = N - r0;
   // M[r0 + q][r0 + i] of the block-start matrix: the input itself in full storage (full:
@@ -276,7 +277,7 @@ __device__ __forceinline__ void pf_panel_body(const float* __restrict__ M, int N
     const int pl = first_lane(gk != 0u ? (kb == gk) : (lane == 0));
     PfCand& my = cand[t & 1][wave];
     if (lane == pl) {
-      my.key = gk;
+      candk[t & 1][wave] = gk;
       my.row = R * tid + ib;
       // the winning slot's x, position and G row, written straight from that slot
 #pragma unroll
@@ -291,12 +292,7 @@ __device__ __forceinline__ void pf_panel_body(const float* __restrict__ M, int N
       }
     }
     __syncthreads();
-    unsigned best = cand[t & 1][0].key;
-    int wb = 0;
-    for (int w = 1; w < NW; ++w) {
-      const unsigned kw = cand[t & 1][w].key;
-      if (kw > best) { best = kw; wb = w; }
-    }
+    const int wb = best_wave<NW>(candk[t & 1][lane & (NW - 1)]);
     const PfCand& win = cand[t & 1][wb];
     const int qp = win.row, pp = win.pos;
     const float d = -win.xv;  // M[a][p] = -M[p][a]
