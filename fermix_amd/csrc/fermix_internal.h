@@ -130,11 +130,13 @@ size_t pf_large_workspace(int64_t batch, int n, bool fact);
 int launch_pf_large(const float* A, int n, int skew, int64_t batch, float* sign, float* logabs,
                     float* gbuf, float* dout, int* perm, void* ws, size_t ws_bytes, hipStream_t s);
 
-// In-place unit-lower (and upper) triangular inverses of a packed (B, Ninv, Ninv) buffer;
-// with active != nullptr only the members with active[b] != 0 are processed.
-int launch_tri_inverse(float* T, int Ninv, int64_t batch, float* Tmp, bool upper, hipStream_t s,
+// In-place unit-lower (and upper) triangular inverses of a packed (B, Ninv, Ninv) buffer that
+// is the identity from order N on (Ninv / 2 < N <= Ninv, Ninv >= 256); with active !=
+// nullptr only the members with active[b] != 0 are processed. Tmp and, with upper, Tmp2
+// hold B * Ninv^2 / 4 floats each (Tmp2: the upper factor's, which may run beside the lower).
+int launch_tri_inverse(float* T, int Ninv, int N, int64_t batch, float* Tmp, float* Tmp2, bool upper, hipStream_t s,
                        const int* active = nullptr, int x3 = 0);
-int launch_unit_lower_inverse(float* T, int Ninv, int64_t batch, float* Tmp, hipStream_t s,
+int launch_unit_lower_inverse(float* T, int Ninv, int N, int64_t batch, float* Tmp, hipStream_t s,
                               const int* active = nullptr, int x3 = 0);
 
 // S^-1 (adjugate = 0) or pf(S) S^-1 (adjugate != 0) as (B, n, n) from the Parlett-Reid
@@ -191,6 +193,9 @@ struct GemmDesc {
   // Optional row transform of B (maskB must be MASK_NONE, transB 0): op(B) row k is
   // s_k B[k ^ 1] with s_k = bscale[b][k / 2], negated for odd k (bscale (batch, K / 2)).
   const float* bscale;
+  // With lim_step > 0 the tiles that start at or past row rlim - z lim_step, or column clim -
+  // z lim_step, of the second batch index z are left out (C keeps what it holds there).
+  int rlim, clim, lim_step;
 };
 
 // C = alpha op(A) op(B) + beta C for every (batch, second-batch) index.

@@ -104,6 +104,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmDesc d) {
     tj = tx % ntn;
   }
   const int i0 = ti * BM, j0 = tj * BN;
+  if (d.lim_step > 0 && (i0 >= d.rlim - (int)bat2 * d.lim_step || j0 >= d.clim - (int)bat2 * d.lim_step)) return;
   const float* A = d.A + bat * d.sA + bat2 * d.sA2;
   const float* B = d.B + bat * d.sB + bat2 * d.sB2;
   float* C = d.C + bat * d.sC + bat2 * d.sC2;
@@ -472,6 +473,7 @@ __global__ __launch_bounds__(256, X3 ? 2 : 4) void gemm128_kernel(GemmDesc d) {
     tj = tx % ntn;
   }
   const int i0 = ti * BM, j0 = tj * BN;
+  if (d.lim_step > 0 && (i0 >= d.rlim - (int)bat2 * d.lim_step || j0 >= d.clim - (int)bat2 * d.lim_step)) return;
   const float* A = d.A + bat * d.sA + bat2 * d.sA2;
   const float* B = d.B + bat * d.sB + bat2 * d.sB2;
   float* C = d.C + bat * d.sC + bat2 * d.sC2;

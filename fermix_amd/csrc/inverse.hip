@@ -216,112 +216,74 @@ __global__ __launch_bounds__(256) void zero_bad_kernel(const int* __restrict__ b
 }
 
 // In-place inverses of the unit-lower L (strictly lower part) and, with upper, of the
-// upper U~ (upper part incl. diagonal) packed in T (B, Ninv, Ninv); Tmp holds
-// B * Ninv^2 / 4 floats.
-int launch_tri_inverse(float* T, int Ninv, int64_t batch, float* Tmp, bool upper, hipStream_t s,
+// upper U~ (upper part incl. diagonal) packed in T (B, Ninv, Ninv), the identity from order N
+// on: the diagonal blocks and tiles past N are left as they are. The two factors' levels are
+// independent: where a level leaves the chip partly idle the upper one's run on the side
+// stream (one level's products are 128 x 128 tiles of about 30 us each, alone on a CU or
+// not). Measured, slogdet + gradient: B = 95, n = 354 867 -> 751 us, B = 30, n = 700 1628 ->
+// 1411, B = 8, n = 900 1732 -> 1609; from 512 tiles per level on one stream serves as well.
+int launch_tri_inverse(float* T, int Ninv, int N, int64_t batch, float* Tmp, float* Tmp2, bool upper, hipStream_t s,
                        const int* active, int x3) {
   const int64_t NN = (int64_t)Ninv * Ninv;
   constexpr int D = 128;  // diagonal blocks inverted whole in LDS
-  hipLaunchKernelGGL((diag_inverse_kernel<D>), dim3(Ninv / D, (unsigned)batch), dim3(256), 0, s, T, Ninv, active,
-                     (int)upper);
+  hipLaunchKernelGGL((diag_inverse_kernel<D>), dim3((N + D - 1) / D, (unsigned)batch), dim3(256), 0, s, T, Ninv,
+                     active, (int)upper);
   if (hipGetLastError() != hipSuccess) return FX_ERR_LAUNCH;
-  for (int sz = D; sz < Ninv; sz *= 2) {
+  SideStream side(s, upper && !active && batch * (Ninv / 256) * (Ninv / 256) <= 512);
+  if (side.ok() && side.fork() != FX_OK) return FX_ERR_LAUNCH;
+  // C (sz x sz, all pairs of a level) = alpha op(A) op(B)
+  auto product = [&](const float* A, int maskA, bool tmpA, const float* B, int maskB, bool tmpB, float* C, bool tmpC,
+                     float alpha, int sz, bool rows, hipStream_t st) {
     const int pairs = Ninv / (2 * sz);
     const int64_t dstride = (int64_t)2 * sz * (Ninv + 1);  // next pair along the diagonal
+    const int64_t tall = (int64_t)pairs * sz * sz, tone = (int64_t)sz * sz;
     GemmDesc d = {};
     d.active = active;
     d.x3 = x3;
     d.M = d.N = d.K = sz;
-    d.sA = d.sB = NN;
-    d.sC = NN;
-    d.lda = d.ldb = d.ldc = Ninv;
-    // L: Tmp = L21 * X11
-    d.A = T + (int64_t)sz * Ninv;
-    d.B = T;
-    d.maskB = MASK_LOWER_UNIT;
-    d.C = Tmp;
-    d.ldc = sz;
-    d.sC = (int64_t)pairs * sz * sz;
-    d.sA2 = d.sB2 = dstride;
-    d.sC2 = (int64_t)sz * sz;
-    d.alpha = 1.0f;
+    d.A = A;
+    d.maskA = maskA;
+    d.lda = tmpA ? sz : Ninv;
+    d.sA = tmpA ? tall : NN;
+    d.sA2 = tmpA ? tone : dstride;
+    d.B = B;
+    d.maskB = maskB;
+    d.ldb = tmpB ? sz : Ninv;
+    d.sB = tmpB ? tall : NN;
+    d.sB2 = tmpB ? tone : dstride;
+    d.C = C;
+    d.ldc = tmpC ? sz : Ninv;
+    d.sC = tmpC ? tall : NN;
+    d.sC2 = tmpC ? tone : dstride;
+    d.alpha = alpha;
     d.beta = 0.0f;
-    int st = launch_gemm(d, batch, pairs, s);
-    if (st != FX_OK) return st;
-    // X21 = -X22 * Tmp
-    GemmDesc e = {};
-    e.active = active;
-    e.x3 = x3;
-    e.M = e.N = e.K = sz;
-    e.A = T + (int64_t)sz * Ninv + sz;
-    e.maskA = MASK_LOWER_UNIT;
-    e.lda = Ninv;
-    e.sA = NN;
-    e.sA2 = dstride;
-    e.B = Tmp;
-    e.ldb = sz;
-    e.sB = (int64_t)pairs * sz * sz;
-    e.sB2 = (int64_t)sz * sz;
-    e.C = T + (int64_t)sz * Ninv;
-    e.ldc = Ninv;
-    e.sC = NN;
-    e.sC2 = dstride;
-    e.alpha = -1.0f;
-    e.beta = 0.0f;
-    st = launch_gemm(e, batch, pairs, s);
+    // rows (L) or columns (U) sz .. of a pair's block that lie past N
+    d.rlim = rows ? N - sz : 1 << 30;
+    d.clim = rows ? 1 << 30 : N - sz;
+    d.lim_step = 2 * sz;
+    return launch_gemm(d, batch, pairs, st);
+  };
+  for (int sz = D; sz < Ninv; sz *= 2) {
+    float* const T21 = T + (int64_t)sz * Ninv;
+    float* const T12 = T + sz;
+    float* const T22 = T21 + sz;
+    // L: Tmp = L21 X11, X21 = -X22 Tmp
+    int st = product(T21, MASK_NONE, false, T, MASK_LOWER_UNIT, false, Tmp, true, 1.0f, sz, true, s);
+    if (st == FX_OK) st = product(T22, MASK_LOWER_UNIT, false, Tmp, MASK_NONE, true, T21, false, -1.0f, sz, true, s);
     if (st != FX_OK) return st;
     if (!upper) continue;
-    // U: Tmp = U12 * Y22
-    GemmDesc f = {};
-    f.active = active;
-    f.x3 = x3;
-    f.M = f.N = f.K = sz;
-    f.A = T + sz;
-    f.lda = Ninv;
-    f.sA = NN;
-    f.sA2 = dstride;
-    f.B = T + (int64_t)sz * Ninv + sz;
-    f.maskB = MASK_UPPER;
-    f.ldb = Ninv;
-    f.sB = NN;
-    f.sB2 = dstride;
-    f.C = Tmp;
-    f.ldc = sz;
-    f.sC = (int64_t)pairs * sz * sz;
-    f.sC2 = (int64_t)sz * sz;
-    f.alpha = 1.0f;
-    f.beta = 0.0f;
-    st = launch_gemm(f, batch, pairs, s);
-    if (st != FX_OK) return st;
-    // Y12 = -Y11 * Tmp
-    GemmDesc h = {};
-    h.active = active;
-    h.x3 = x3;
-    h.M = h.N = h.K = sz;
-    h.A = T;
-    h.maskA = MASK_UPPER;
-    h.lda = Ninv;
-    h.sA = NN;
-    h.sA2 = dstride;
-    h.B = Tmp;
-    h.ldb = sz;
-    h.sB = (int64_t)pairs * sz * sz;
-    h.sB2 = (int64_t)sz * sz;
-    h.C = T + sz;
-    h.ldc = Ninv;
-    h.sC = NN;
-    h.sC2 = dstride;
-    h.alpha = -1.0f;
-    h.beta = 0.0f;
-    st = launch_gemm(h, batch, pairs, s);
+    // U: Tmp2 = U12 Y22, Y12 = -Y11 Tmp2
+    const hipStream_t su = side.side();
+    st = product(T12, MASK_NONE, false, T22, MASK_UPPER, false, Tmp2, true, 1.0f, sz, false, su);
+    if (st == FX_OK) st = product(T, MASK_UPPER, false, Tmp2, MASK_NONE, true, T12, false, -1.0f, sz, false, su);
     if (st != FX_OK) return st;
   }
-  return FX_OK;
+  return side.join();
 }
 
-int launch_unit_lower_inverse(float* T, int Ninv, int64_t batch, float* Tmp, hipStream_t s,
+int launch_unit_lower_inverse(float* T, int Ninv, int N, int64_t batch, float* Tmp, hipStream_t s,
                               const int* active, int x3) {
-  return launch_tri_inverse(T, Ninv, batch, Tmp, false, s, active, x3);
+  return launch_tri_inverse(T, Ninv, N, batch, Tmp, nullptr, false, s, active, x3);
 }
 
 int inv_padded(int N) {
@@ -368,15 +330,15 @@ int launch_lu_inverse(float* LU, const int* g0, int N, int n, int64_t batch, con
                        LU, N, T, Ninv);
     if (hipGetLastError() != hipSuccess) return FX_ERR_LAUNCH;
   }
-  int st0 = launch_tri_inverse(T, Ninv, batch, Tmp, true, s, nullptr, x3);
+  // the output, unused so far and at least Ninv^2 / 4 floats a member (n > Ninv / 2), holds Tmp2
+  int st0 = launch_tri_inverse(T, Ninv, N, batch, Tmp, invT, true, s, nullptr, x3);
   if (st0 != FX_OK) return st0;
   // Z = U~^-1 L^-1 (the leading N x N block) stored straight as invT = P^T Z^T:
   // invT[g0[c]][i] = Z[i][c] for i < n and g0[c] < n, with the non-finite tile flags
   {
     GemmDesc d = {};
     d.x3 = x3;
-    d.M = d.N = N;
-    d.K = Ninv;
+    d.M = d.N = d.K = N;
     d.A = T;
     d.maskA = MASK_UPPER;
     d.B = T;

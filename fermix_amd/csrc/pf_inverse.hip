@@ -327,7 +327,7 @@ int launch_pf_inverse(const float* gbuf, int PB, const float* d, const int* perm
     hipLaunchKernelGGL(pf_assemble_kernel, dim3((unsigned)Ninv, (unsigned)batch), dim3(256), 0, s, gbuf, PB, N,
                        perm, dinv, T, Ninv, active);
     if (hipGetLastError() != hipSuccess) return FX_ERR_LAUNCH;
-    int st = launch_unit_lower_inverse(T, Ninv, batch, Tmp, s, active, x3);
+    int st = launch_unit_lower_inverse(T, Ninv, N, batch, Tmp, s, active, x3);
     if (st != FX_OK) return st;
     {
       // R = Y^T DY: op(A) = Y^T (upper, unit diagonal), lower tiles, mirrored skew
