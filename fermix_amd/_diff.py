@@ -41,39 +41,50 @@ from ._kernels import DEFAULT_X3
 _functorch = getattr(torch._C, "_functorch", None)
 
 
+def _wrapped(A):
+    return _functorch is not None and _functorch.is_functorch_wrapped_tensor(A)
+
+
+def _dual(A):
+    try:
+        return fwAD.unpack_dual(A).tangent is not None
+    except Exception:  # pragma: no cover - no dual level active
+        return False
+
+
 def _plain(A):
-    """Neither a forward-mode dual nor a torch.func wrapper, and not under a tracer or a
+    """No torch.func transform active, no forward-mode dual, and not under a tracer or a
     compiler (which record the autograd functions): what happens to A can only be eager
-    reverse mode, or nothing."""
-    if _functorch is not None and _functorch.is_functorch_wrapped_tensor(A):
+    reverse mode, or nothing. A transform counts also where A is closed over and not
+    wrapped: under it torch refuses functions without setup_context, and the tensors that a
+    kernel call would allocate are the transform's wrappers, so such a call goes through the
+    functions that torch lowers to the level of A."""
+    if torch._C._are_functorch_transforms_active() or _wrapped(A):
         return False
     if torch.jit.is_tracing() or torch.compiler.is_compiling():
         return False
-    try:
-        return fwAD.unpack_dual(A).tangent is None
-    except Exception:  # pragma: no cover - no dual level active
-        return True
+    return not _dual(A)
 
 
 def _wants_grad(A):
     """Whether a derivative of this call can be requested: autograd tracking, a
     forward-mode dual, or a torch.func grad/jvp wrapper around the input."""
-    if A.requires_grad:
+    if A.requires_grad or _dual(A):
         return True
-    try:
-        if fwAD.unpack_dual(A).tangent is not None:
-            return True
-    except Exception:  # pragma: no cover - no dual level active
-        pass
-    if _functorch is not None and _functorch.is_functorch_wrapped_tensor(A):
-        return not _functorch.is_batchedtensor(A)
-    return False
+    return _wrapped(A) and not _functorch.is_batchedtensor(A)
+
+
+def _plain_reverse(A):
+    """A plain autograd tensor (requires_grad, no forward-mode dual, no torch.func
+    wrapper): its derivative can only come from a backward pass on real tensors, so
+    the factors may be kept and the inverse formed in the backward."""
+    return A.requires_grad and not _dual(A) and not _wrapped(A)
 
 
 class _Reverse(torch.autograd.Function):
-    """Plain eager reverse mode of a rule: rule.forward(A, *args) -> (outputs, saved) and
-    rule.backward(ctx, *cotangents) -> the gradient of A. What a rule saves need not be an
-    output here (torch.func's functions, below, can only save inputs and outputs), so a call
+    """Eager reverse mode of a rule where _plain holds: rule.forward(A, *args) -> (outputs,
+    saved) and rule.backward(ctx, *cotangents) -> the gradient of A. What a rule saves need
+    not be an output here (torch.func's functions, below, can only save inputs and outputs), so a call
     hands autograd the values alone: 40 -> 21 us of host time for slogdet n = 40 (147 -> 50 us
     with its gradient)."""
 
@@ -250,20 +261,62 @@ class _SlogdetPartsRule:
         return _apply_cotangent(_log_cotangent(sign, g_sign, g_logabs), invT)
 
 
+class _SlogdetSplit(torch.autograd.Function):
+    """_SlogdetSplitRule as a function that torch.func and the tracers take (the factors are
+    outputs): a plain autograd tensor closed over inside a transform of something else, or
+    under a tracer. The jvp (real tensors only) forms A^-T from a copy of lu."""
+
+    @staticmethod
+    def forward(A, x3):
+        return _kernels.slogdet_factors(A, x3)
+
+    @staticmethod
+    def setup_context(ctx, inputs, output):
+        sign, logabs, lu, perm = output
+        ctx.mark_non_differentiable(sign, lu, perm)
+        ctx.set_materialize_grads(False)
+        ctx.save_for_backward(inputs[0], sign, lu, perm)
+        ctx.save_for_forward(sign, lu, perm)
+        ctx.n = inputs[0].shape[-1]
+        ctx.args = (inputs[1],)
+        ctx.used = False
+
+    @staticmethod
+    def backward(ctx, g_sign, g_logabs, g_lu, g_perm):
+        if g_logabs is None:
+            return None, None
+        return _SlogdetSplitRule.backward(ctx, g_sign, g_logabs), None
+
+    @staticmethod
+    def jvp(ctx, dA, _x3):
+        sign, lu, perm = ctx.saved_tensors
+        invT = _kernels.slogdet_inverse(lu.clone(), perm, sign, ctx.n, x3=ctx.args[0])
+        dlog = (invT * dA).sum(dim=(-1, -2))
+        return None, dlog, None, None
+
+    @staticmethod
+    def vmap(info, in_dims, A, x3):
+        A2, vb = _fold(info, in_dims[:1], A)
+        out = _SlogdetSplit.apply(A2, x3)
+        if vb is None:
+            return out, (None,) * 4
+        return tuple(_unfold(x, vb) for x in out), (0,) * 4
+
+
 def slogdet(A, x3=DEFAULT_X3):
     """x3: the split-bf16x3 product mode of the blocked kernels (0: fp32 MFMA)."""
-    if _plain(A):
-        if not (A.requires_grad and torch.is_grad_enabled()):
-            return _kernels.slogdet(A, x3)
-        # n <= 32: one Gauss-Jordan pass forms A^-T with the factors
-        n = A.shape[-1]
-        split = (A.dtype == torch.float32 and 32 < n <= _tune.LARGE_MAX_N
-                 and _tune.kernel_family(n, "slogdet") != "generic")
-        return _Reverse.apply(A, _SlogdetSplitRule if split else _SlogdetPartsRule, x3)
+    plain = _plain(A)
+    if plain and not (A.requires_grad and torch.is_grad_enabled()):
+        return _kernels.slogdet(A, x3)
     if _wants_grad(A):
-        # forward mode and torch.func transforms: the parts call (the rules run on wrapped tensors)
-        s, l, _ = _SlogdetParts.apply(A, x3)
-        return s, l
+        # n <= 32: one Gauss-Jordan pass forms A^-T with the factors; forward mode and wrapped
+        # tensors: the parts call (its rules run on them)
+        n = A.shape[-1]
+        split = (A.dtype == torch.float32 and 32 < n <= _tune.LARGE_MAX_N and _plain_reverse(A)
+                 and _tune.kernel_family(n, "slogdet") != "generic")
+        if plain:
+            return _Reverse.apply(A, _SlogdetSplitRule if split else _SlogdetPartsRule, x3)
+        return (_SlogdetSplit if split else _SlogdetParts).apply(A, x3)[:2]
     return _SlogdetFwd.apply(A, x3)
 
 
@@ -354,19 +407,59 @@ class _SlogpfPartsRule:
         return _apply_cotangent(-0.5 * _log_cotangent(sign, g_sign, g_logabs), Sinv)
 
 
+class _SlogpfSplit(torch.autograd.Function):
+    """_SlogpfSplitRule as a function that torch.func and the tracers take (see
+    _SlogdetSplit). The jvp (real tensors only) forms S^-1."""
+
+    @staticmethod
+    def forward(A, skew, x3):
+        return _kernels.slogpf_factors(A, skew)
+
+    @staticmethod
+    def setup_context(ctx, inputs, output):
+        sign, logabs, gbuf, d, perm = output
+        ctx.mark_non_differentiable(sign, gbuf, d, perm)
+        ctx.set_materialize_grads(False)
+        ctx.save_for_backward(gbuf, d, perm)
+        ctx.save_for_forward(gbuf, d, perm)
+        ctx.n = inputs[0].shape[-1]
+        ctx.args = (inputs[1], inputs[2])
+
+    @staticmethod
+    def backward(ctx, g_sign, g_logabs, g_gbuf, g_d, g_perm):
+        if g_logabs is None:
+            return None, None, None
+        return _SlogpfSplitRule.backward(ctx, g_sign, g_logabs), None, None
+
+    @staticmethod
+    def jvp(ctx, dA, _skew, _x3):
+        gbuf, d, perm = ctx.saved_tensors
+        Sinv = _kernels.slogpf_inverse(gbuf, d, perm, ctx.n, x3=ctx.args[1])
+        dlog = -0.5 * (Sinv * dA).sum(dim=(-1, -2))
+        return None, dlog, None, None, None
+
+    @staticmethod
+    def vmap(info, in_dims, A, skew, x3):
+        A2, vb = _fold(info, in_dims[:1], A)
+        out = _SlogpfSplit.apply(A2, skew, x3)
+        if vb is None:
+            return out, (None,) * 5
+        return tuple(_unfold(x, vb) for x in out), (0,) * 5
+
+
 def slogpf(A, skew, x3=DEFAULT_X3):
     """x3: the split-bf16x3 product mode of the gradient's GEMMs (the forward's trailing
     update is memory-bound and runs in fp32 in both modes)."""
-    if _plain(A):
-        if not (A.requires_grad and torch.is_grad_enabled()):
-            return _kernels.slogpf(A, skew, x3=x3)
-        n = A.shape[-1]
-        split = (A.dtype == torch.float32 and 0 < n <= _tune.LARGE_MAX_N and n % 2 == 0
-                 and _tune.kernel_family(n, "slogpf") != "generic")
-        return _Reverse.apply(A, _SlogpfSplitRule if split else _SlogpfPartsRule, skew, x3)
+    plain = _plain(A)
+    if plain and not (A.requires_grad and torch.is_grad_enabled()):
+        return _kernels.slogpf(A, skew, x3=x3)
     if _wants_grad(A):
-        s, l, _ = _SlogpfParts.apply(A, skew, x3)
-        return s, l
+        n = A.shape[-1]
+        split = (A.dtype == torch.float32 and 0 < n <= _tune.LARGE_MAX_N and n % 2 == 0 and _plain_reverse(A)
+                 and _tune.kernel_family(n, "slogpf") != "generic")
+        if plain:
+            return _Reverse.apply(A, _SlogpfSplitRule if split else _SlogpfPartsRule, skew, x3)
+        return (_SlogpfSplit if split else _SlogpfParts).apply(A, skew, x3)[:2]
     return _SlogpfFwd.apply(A, skew, x3)
 
 
