@@ -109,3 +109,25 @@ def test_pr(dev, kind, n):
     Bt = torch.from_numpy(np.ascontiguousarray(_grid(S))).to(dev)
     for got, want in zip(_kernels.slogpf_parts(At, True), _kernels.slogpf_parts(Bt, False)):
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("n", [16, 32, 33, 64, 65, 128])
+def test_det_scale_c64(dev, n):
+    """adj(A)^T = det A^-T with the det that the factorisation holds in double: of diagonal
+    matrices of 2, -2, 2i, 1 the inverse and the adjugate are exact in complex64, and one
+    rounding (2^-23 with the exp and the product) is left. A logabs rounded to float32 alone
+    would give up to 2^-25 logabs, 1.3e-6 at n = 64."""
+    rng = np.random.default_rng(9400 + n)
+    d = rng.choice(np.array([2, -2, 2j, 1]), (24, n))
+    A = np.zeros((24, n, n), np.complex64)
+    A[:, np.arange(n), np.arange(n)] = d
+    order = rng.permutation(n)
+    A = A[:, order]
+    print(f"field_small det scale n={n}", flush=True)
+    adj = _np(_kernels.det_parts(torch.from_numpy(A).to(dev))[2])
+    det = np.prod(d, axis=1) * np.linalg.det(np.eye(n)[order])
+    ref = np.zeros(A.shape, np.complex128)
+    ref[:, np.arange(n), order] = det[:, None] / d[:, order]
+    assert np.all(adj[ref == 0] == 0)
+    err = np.abs(adj[ref != 0] - ref[ref != 0]) / np.abs(ref[ref != 0])
+    assert np.max(err) <= 2.0**-23, np.max(err)
