@@ -59,11 +59,9 @@ def _plain(A):
     wrapped: under it torch refuses functions without setup_context, and the tensors that a
     kernel call would allocate are the transform's wrappers, so such a call goes through the
     functions that torch lowers to the level of A."""
-    if torch._C._are_functorch_transforms_active() or _wrapped(A):
+    if torch._C._are_functorch_transforms_active() or torch.jit.is_tracing() or torch.compiler.is_compiling():
         return False
-    if torch.jit.is_tracing() or torch.compiler.is_compiling():
-        return False
-    return not _dual(A)
+    return not (_wrapped(A) or _dual(A))
 
 
 def _wants_grad(A):
@@ -303,20 +301,24 @@ class _SlogdetSplit(torch.autograd.Function):
         return tuple(_unfold(x, vb) for x in out), (0,) * 4
 
 
+def _slogdet_split(A):
+    """Whether a gradient call keeps the factors. n <= 32: one Gauss-Jordan pass forms A^-T
+    with them."""
+    n = A.shape[-1]
+    return (A.dtype == torch.float32 and 32 < n <= _tune.LARGE_MAX_N
+            and _tune.kernel_family(n, "slogdet") != "generic")
+
+
 def slogdet(A, x3=DEFAULT_X3):
     """x3: the split-bf16x3 product mode of the blocked kernels (0: fp32 MFMA)."""
-    plain = _plain(A)
-    if plain and not (A.requires_grad and torch.is_grad_enabled()):
-        return _kernels.slogdet(A, x3)
+    if _plain(A):
+        if not (A.requires_grad and torch.is_grad_enabled()):
+            return _kernels.slogdet(A, x3)
+        return _Reverse.apply(A, _SlogdetSplitRule if _slogdet_split(A) else _SlogdetPartsRule, x3)
     if _wants_grad(A):
-        # n <= 32: one Gauss-Jordan pass forms A^-T with the factors; forward mode and wrapped
-        # tensors: the parts call (its rules run on them)
-        n = A.shape[-1]
-        split = (A.dtype == torch.float32 and 32 < n <= _tune.LARGE_MAX_N and _plain_reverse(A)
-                 and _tune.kernel_family(n, "slogdet") != "generic")
-        if plain:
-            return _Reverse.apply(A, _SlogdetSplitRule if split else _SlogdetPartsRule, x3)
-        return (_SlogdetSplit if split else _SlogdetParts).apply(A, x3)[:2]
+        # forward mode and wrapped tensors: the parts call (its rules run on them)
+        f = _SlogdetSplit if _plain_reverse(A) and _slogdet_split(A) else _SlogdetParts
+        return f.apply(A, x3)[:2]
     return _SlogdetFwd.apply(A, x3)
 
 
@@ -447,19 +449,23 @@ class _SlogpfSplit(torch.autograd.Function):
         return tuple(_unfold(x, vb) for x in out), (0,) * 5
 
 
+def _slogpf_split(A):
+    """Whether a gradient call keeps the factors."""
+    n = A.shape[-1]
+    return (A.dtype == torch.float32 and 0 < n <= _tune.LARGE_MAX_N and n % 2 == 0
+            and _tune.kernel_family(n, "slogpf") != "generic")
+
+
 def slogpf(A, skew, x3=DEFAULT_X3):
     """x3: the split-bf16x3 product mode of the gradient's GEMMs (the forward's trailing
     update is memory-bound and runs in fp32 in both modes)."""
-    plain = _plain(A)
-    if plain and not (A.requires_grad and torch.is_grad_enabled()):
-        return _kernels.slogpf(A, skew, x3=x3)
+    if _plain(A):
+        if not (A.requires_grad and torch.is_grad_enabled()):
+            return _kernels.slogpf(A, skew, x3=x3)
+        return _Reverse.apply(A, _SlogpfSplitRule if _slogpf_split(A) else _SlogpfPartsRule, skew, x3)
     if _wants_grad(A):
-        n = A.shape[-1]
-        split = (A.dtype == torch.float32 and 0 < n <= _tune.LARGE_MAX_N and n % 2 == 0 and _plain_reverse(A)
-                 and _tune.kernel_family(n, "slogpf") != "generic")
-        if plain:
-            return _Reverse.apply(A, _SlogpfSplitRule if split else _SlogpfPartsRule, skew, x3)
-        return (_SlogpfSplit if split else _SlogpfParts).apply(A, skew, x3)[:2]
+        f = _SlogpfSplit if _plain_reverse(A) and _slogpf_split(A) else _SlogpfParts
+        return f.apply(A, skew, x3)[:2]
     return _SlogpfFwd.apply(A, skew, x3)
 
 
