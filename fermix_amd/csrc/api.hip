@@ -400,7 +400,7 @@ int fx_det_parts_f32(const float* a, int64_t batch, int32_t n, float* sign, floa
       p += align256(wl);
     }
     if (st != FX_OK) return st;
-    if (N <= SMALL_INV_MAXN) return launch_lu_inv_small(LU, g0, N, n, nb, sg, lg, nullptr, 0, true, adj, s);
+    if (N <= SMALL_INV_MAXN) return launch_lu_inv_small(LU, g0, N, n, nb, sg, nullptr, 0, true, adj, s);
     // the adjugate's scalars and vectors come from the LU before the inverse overwrites it
     void* dws = p;
     p += align256(det_adjugate_workspace(nb, n));

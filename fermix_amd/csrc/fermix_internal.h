@@ -112,12 +112,11 @@ int launch_lu_inverse(float* LU, const int* g0, int N, int n, int64_t batch, con
 
 // The same from padded orders N <= SMALL_INV_MAXN (a multiple of 16) in one launch each, read
 // only, no workspace (small_inverse.hip): launch_lu_inverse's A^-T or, with det, adj(A)^T =
-// d det / dA (sign / logabs the factorisation's own; scale unused), and launch_pf_inverse's
+// d det / dA (sign the factorisation's own; scale unused), and launch_pf_inverse's
 // results.
 constexpr int SMALL_INV_MAXN = 128;
 int launch_lu_inv_small(const float* LU, const int* g0, int N, int n, int64_t batch, const float* sign,
-                        const float* logabs, const float* scale, int zero_singular, bool det, float* out,
-                        hipStream_t s);
+                        const float* scale, int zero_singular, bool det, float* out, hipStream_t s);
 int launch_pf_inv_small(const float* gbuf, int PB, const float* d, const int* perm, int N, int n, int64_t batch,
                         int adjugate, const float* scale, float* out, hipStream_t s);
 

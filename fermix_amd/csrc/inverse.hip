@@ -312,7 +312,7 @@ int launch_lu_inverse(float* LU, const int* g0, int N, int n, int64_t batch, con
   const bool need_copy = !(in_place && Ninv == N);
   if (!ws || ws_bytes < lu_inverse_workspace(batch, N, need_copy)) return FX_ERR_WORKSPACE;
   if (N <= SMALL_INV_MAXN)
-    return launch_lu_inv_small(LU, g0, N, n, batch, sign, nullptr, scale, zero_singular, false, invT, s);
+    return launch_lu_inv_small(LU, g0, N, n, batch, sign, scale, zero_singular, false, invT, s);
   char* p = (char*)ws;
   auto take = [&](size_t x) {
     char* q = p;
