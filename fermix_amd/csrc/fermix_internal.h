@@ -3,8 +3,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <mutex>
-
 #include "../../include/fermix.h"
 
 namespace fx {
@@ -24,29 +22,27 @@ struct TunePin {
   bool own_;
 };
 
-// The device's second stream (side.hip) for a driver that runs two halves of a batch side
-// by side. With want and the stream available (not under graph capture), ok() holds and
-// the device's side stream is reserved until the destructor: fork() orders the side
-// stream after the work enqueued so far on s, join() (also run by the destructor) orders
-// s after the side stream's work.
+// A second stream (side.hip) for a driver that runs two parts of a call side by side. With want
+// and one available (not under graph capture), ok() holds and the side stream is this
+// object's until the destructor: fork() orders it after the work enqueued so far on s,
+// join() (also run by the destructor) orders s after its work.
+struct SideSlot;
 class SideStream {
  public:
   SideStream(hipStream_t s, bool want);
   ~SideStream();
   SideStream(const SideStream&) = delete;
   SideStream& operator=(const SideStream&) = delete;
-  bool ok() const { return side_ != nullptr; }
-  hipStream_t side() const { return side_ ? *side_ : s_; }
+  bool ok() const { return slot_ != nullptr; }
+  hipStream_t side() const;
   int fork();
   int join();
 
  private:
   hipStream_t s_;
-  hipStream_t* side_ = nullptr;
-  hipEvent_t* fork_ = nullptr;
-  hipEvent_t* join_ = nullptr;
+  SideSlot* slot_ = nullptr;
+  int dev_ = -1;
   bool forked_ = false;
-  std::unique_lock<std::mutex> lk_;
 };
 
 // Compute units of the current device (side.hip; queried once per device, 256 if the
@@ -204,12 +200,13 @@ int launch_gemm(const GemmDesc& d, int64_t batch, int nb2, hipStream_t s);
 // determinant with det), zero for singular members
 int launch_lu64_small(const double* a, int n, int64_t batch, double* sign, double* logabs, double* out, bool det,
                       hipStream_t s);
-// Whether a parts run's Parlett-Reid goes beside its LU on the side stream: both are chains of
+// Whether a parts run's Parlett-Reid goes beside its LU on a side stream: both are chains of
 // panels on one workgroup per matrix that leave most of a CU idle. slogpf + S^-1, alone ->
-// beside, us: float64 B = 48, n = 302 1950 -> 1395, B = 200, n = 302 3286 -> 2846, B = 512, n =
-// 200 2919 -> 2794, B = 1000, n = 140 2644 -> 2576; the gain fades with the batch, so not above
-// 1024. Not above n = 512, where panels span several cooperatively launched workgroups that
-// must all be resident.
+// beside, us, B = 48 / 200 / 512, n = 302: float64 1882 -> 1384, 3244 -> 2788, 6931 -> 6618,
+// complex64 2594 -> 1917, 4789 -> 4254, 10782 -> 10412, complex128 3460 -> 2419, 6955 -> 6329,
+// 15987 -> 15619; B = 1024, n = 130: 2556 -> 2475, 3590 -> 3516, 6362 -> 6285. The gain fades with
+// the batch, so not above 1024. Not above n = 512, where panels span several cooperatively
+// launched workgroups that must all be resident.
 inline bool pf_parts_overlap(int64_t batch, int n) { return n <= 512 && batch <= 1024; }
 // float64 blocked LU (sign, logabs) for the orders above the register kernels (lu64_impl.inc)
 size_t lu64_workspace(int64_t batch, int n);

@@ -1,13 +1,18 @@
-// A second stream per device for the blocked drivers that run two halves of a batch side
-// by side (launch_pf_large, launch_lu_large): a half's panel kernels, one latency-bound
-// workgroup per matrix, then run beside the other half's trailing update, which streams
-// the matrices through HBM or keeps the MFMA busy.
+// Second streams for the drivers that run two independent parts of one call side by side:
+//  - launch_lu_large, launch_pf_large: the two halves of a batch, one half's panels (one
+//    latency-bound workgroup per matrix) beside the other's trailing update;
+//  - launch_tri_inverse: the two triangular factors' levels of a small batch;
+//  - the float64 / complex slogpf gradients: the Parlett-Reid beside the LU.
 //
-// The stream is created on first use with hipStreamNonBlocking (no implicit ordering
-// with the null stream; every dependency is an explicit event) at the default priority,
-// and kept, with its two events, until the process ends. A split run holds the
-// device's mutex from its fork to its join, so two host threads never interleave their
-// records of the shared events. A stream under graph capture runs unsplit.
+// A device has up to SIDE_SLOTS side streams, each created when a caller stream first needs one
+// more, with hipStreamNonBlocking (no implicit ordering with the null stream; every
+// dependency is an explicit event) at the default priority, and kept, with its two events,
+// until the process ends. A call takes the slot that its own stream used last, else a fresh
+// one, else the one unused for longest, and holds it from its construction to its
+// destructor, so that no two host threads record the same events. So callers on up to
+// SIDE_SLOTS streams never queue behind each other's side work, and no call waits for
+// another host thread: with every slot held, or under graph capture, it runs unsplit (the
+// same bits).
 #include <atomic>
 #include <mutex>
 
@@ -17,42 +22,71 @@ namespace fx {
 namespace {
 
 constexpr int SIDE_MAXDEV = 64;
+constexpr int SIDE_SLOTS = 4;
 
-struct Side {
-  std::mutex mu;
-  bool tried = false, ok = false;
+}  // namespace
+
+struct SideSlot {
+  bool tried = false, ok = false, held = false;
+  hipStream_t owner = nullptr;  // the caller stream that used it last (tried only)
+  unsigned long long used = 0;  // when
   hipStream_t s2 = nullptr;
   hipEvent_t fork = nullptr, join = nullptr;
 };
 
-Side g_side[SIDE_MAXDEV];
+namespace {
+
+struct SidePool {
+  std::mutex mu;
+  unsigned long long clock = 0;
+  SideSlot slot[SIDE_SLOTS];
+};
+
+SidePool g_side[SIDE_MAXDEV];
+
+// The slot for s, marked as held, or nullptr.
+SideSlot* take_slot(SidePool& p, hipStream_t s) {
+  std::lock_guard<std::mutex> lk(p.mu);
+  SideSlot *own = nullptr, *fresh = nullptr, *oldest = nullptr;
+  for (SideSlot& t : p.slot) {
+    if (t.held) continue;
+    if (!t.tried) {
+      if (!fresh) fresh = &t;
+    } else if (t.ok) {
+      if (t.owner == s) own = &t;
+      if (!oldest || t.used < oldest->used) oldest = &t;
+    }
+  }
+  if (!own && fresh) {
+    fresh->tried = true;
+    fresh->ok = hipStreamCreateWithFlags(&fresh->s2, hipStreamNonBlocking) == hipSuccess &&
+                hipEventCreateWithFlags(&fresh->fork, hipEventDisableTiming) == hipSuccess &&
+                hipEventCreateWithFlags(&fresh->join, hipEventDisableTiming) == hipSuccess;
+    if (!fresh->ok) fresh = nullptr;
+  }
+  SideSlot* t = own ? own : fresh ? fresh : oldest;
+  if (!t) return nullptr;
+  t->held = true;
+  t->owner = s;
+  t->used = ++p.clock;
+  return t;
+}
 
 }  // namespace
 
 SideStream::SideStream(hipStream_t s, bool want) : s_(s) {
   if (!want) return;
-  int dev = -1;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= SIDE_MAXDEV) return;
+  if (hipGetDevice(&dev_) != hipSuccess || dev_ < 0 || dev_ >= SIDE_MAXDEV) return;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return;
-  Side& d = g_side[dev];
-  std::unique_lock<std::mutex> lk(d.mu);
-  if (!d.tried) {
-    d.tried = true;
-    d.ok = hipStreamCreateWithFlags(&d.s2, hipStreamNonBlocking) == hipSuccess &&
-           hipEventCreateWithFlags(&d.fork, hipEventDisableTiming) == hipSuccess &&
-           hipEventCreateWithFlags(&d.join, hipEventDisableTiming) == hipSuccess;
-  }
-  if (!d.ok) return;
-  lk_ = std::move(lk);
-  side_ = &d.s2;
-  fork_ = &d.fork;
-  join_ = &d.join;
+  slot_ = take_slot(g_side[dev_], s);
 }
 
+hipStream_t SideStream::side() const { return slot_ ? slot_->s2 : s_; }
+
 int SideStream::fork() {
-  if (!side_ || forked_) return FX_ERR_LAUNCH;
-  if (hipEventRecord(*fork_, s_) != hipSuccess || hipStreamWaitEvent(*side_, *fork_, 0) != hipSuccess)
+  if (!slot_ || forked_) return FX_ERR_LAUNCH;
+  if (hipEventRecord(slot_->fork, s_) != hipSuccess || hipStreamWaitEvent(slot_->s2, slot_->fork, 0) != hipSuccess)
     return FX_ERR_LAUNCH;
   forked_ = true;
   return FX_OK;
@@ -61,12 +95,17 @@ int SideStream::fork() {
 int SideStream::join() {
   if (!forked_) return FX_OK;
   forked_ = false;
-  if (hipEventRecord(*join_, *side_) != hipSuccess || hipStreamWaitEvent(s_, *join_, 0) != hipSuccess)
+  if (hipEventRecord(slot_->join, slot_->s2) != hipSuccess || hipStreamWaitEvent(s_, slot_->join, 0) != hipSuccess)
     return FX_ERR_LAUNCH;
   return FX_OK;
 }
 
-SideStream::~SideStream() { join(); }
+SideStream::~SideStream() {
+  join();
+  if (!slot_) return;
+  std::lock_guard<std::mutex> lk(g_side[dev_].mu);
+  slot_->held = false;
+}
 
 int device_cus() {
   static std::atomic<int> cache[SIDE_MAXDEV];
