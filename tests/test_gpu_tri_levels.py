@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from fermix_amd import _kernels
+from fermix_amd import _kernels, _lib
 from tests.tolerances import relerr
 
 pytestmark = pytest.mark.gpu
@@ -27,3 +27,28 @@ def test_levels(dev, n, big, x3):
     assert max(relerr(got[k], ref[k]) for k in range(4)) < 1e-4
     many = At.repeat((big + 3) // 4, 1, 1)
     assert torch.equal(_kernels.slogdet_parts(many, x3=x3)[2][-4:], inv)
+
+
+@pytest.mark.parametrize("n", [129, 193, 300, 520, 700, 1100])
+@pytest.mark.parametrize("x3", [0, 1])
+def test_stale_workspace(dev, n, x3):
+    """The tiles that are left out stay unwritten in the workspace and in the output, which
+    holds the upper factor's intermediate: the same bits over stale NaN as over zeros, with
+    64- and 128-wide tiles (fp32 products take the wide ones from level 512 on)."""
+    rng = np.random.default_rng(9350 + n)
+    B = 3
+    A = (np.eye(n) + 0.5 * rng.standard_normal((B, n, n)) / np.sqrt(n)).astype(np.float32)[:, rng.permutation(n)]
+    print(f"stale workspace n={n} x3={x3}", flush=True)
+    sign, _, lu0, perm = _kernels.slogdet_factors(torch.from_numpy(np.ascontiguousarray(A)).to(dev), x3)
+    L = _lib.lib()
+    wsb = L.fx_slogdet_inverse_f32_workspace(B, n)
+    got = []
+    for stale in (0.0, float("nan")):
+        lu = lu0.clone()
+        ws = torch.full((wsb // 4,), stale, device=dev)
+        out = torch.full((B, n, n), stale, device=dev)
+        st = L.fx_slogdet_inverse_f32(lu.data_ptr(), perm.data_ptr(), sign.data_ptr(), None, B, n, 1, out.data_ptr(), x3,
+                                      ws.data_ptr(), wsb, torch.cuda.current_stream().cuda_stream or None)
+        assert st == 0
+        got.append(out)
+    assert bool(torch.isfinite(got[0]).all()) and bool((got[0] != 0).any()) and torch.equal(*got)
