@@ -21,8 +21,9 @@ float64 and complex inputs, and float32 where the field-generic kernels run (the
 fx_tune.lu_generic_above_n, everything above 8192; no packed factors are exported
 there), take the parts route (A^-T / S^-1 formed with the
 primal by the field-generic blocked kernels); for complex kinds the sign is differentiable too, with
-the reference's conventions (see _log_tangents below). Their det derivative is the exact
-adjugate of the same Gauss-Jordan run (fx_det_parts_f64 / _c64 / _c128); their pf
+the reference's conventions (see _log_tangents below). Their det derivative is the adjugate of
+fx_det_parts_f64 / _c64 / _c128 (det A^-T of the forward's LU, for exactly singular members
+a Gauss-Jordan run's continuation); their pf
 derivative is the Pfaffian adjugate of fx_slogpf_parts_f64 / _c64 / _c128 (adjugate
 mode), with the primal from the plain forward's own kernel. For complex kinds the
 backward applies torch's conjugate convention (cotangent times the conjugate of the

@@ -54,7 +54,7 @@ __device__ __forceinline__ void cload(const F* __restrict__ a, int n, int skew, 
   }
 }
 
-enum { GJ_ADJ = 2, GJ_PFA = 3 };
+enum { GJ_ADJ, GJ_PFA };
 
 // ---- the Pfaffian adjugate pf(S) S^-1 (the pf gradient) of the 64-bit and complex kinds.
 // Parlett-Reid with the rows and columns permuted (P), P S P^T = L D L^T with D = diag_s(
@@ -514,10 +514,10 @@ int cx_empty(void* sign, void* logabs, int64_t batch, hipStream_t s) {
 // The LU (values; with the inverse) and the Parlett-Reid of a field: the matrix in LDS where
 // field_small.inc covers the order (no workspace), else the blocked kernels. The orders
 // follow from what 160 KiB hold. Measured, us, slogdet / + gradient / slogpf / + gradient:
-//   complex64  B = 1024, n = 64   853 / 1256 / 435 / 1701 -> 48 / 147 / 49 / 212
-//   complex64  B = 1024, n = 100  915 / 1791 / 1192 / 3040 -> 465 / 623 / 264 / 917
-//   complex128 B = 1024, n = 64   1311 / 1857 / 744 / 2621 -> 113 / 207 / 99 / 321
-//   complex128 B = 1024, n = 96   1189 / 2039 / 1488 / 3576 -> 529 / 718 / 387 / 1126
+//   complex64  B = 1024, n = 64   853 / 1256 / 435 / 1701 -> 51 / 155 / 52 / 214
+//   complex64  B = 1024, n = 100  915 / 1791 / 1192 / 3040 -> 460 / 630 / 265 / 925
+//   complex128 B = 1024, n = 64   1311 / 1857 / 744 / 2621 -> 117 / 210 / 103 / 329
+//   complex128 B = 1024, n = 96   1189 / 2039 / 1488 / 3576 -> 557 / 745 / 400 / 1168
 // (before: one unblocked workgroup of 1024 threads for n <= 64, the blocked kernels above).
 template <class F>
 bool lds_lu(int n) {
@@ -829,7 +829,7 @@ int slogpf_parts(const T* a, int64_t batch, int n, int skew, int adjugate, T* si
 }  // namespace
 
 // the float64 Pfaffian adjugate (fx_slogpf_parts_f64 with adjugate != 0): zero for odd n.
-// Above the register kernels (n > f64_reg_max_n) the members the gate passes (pf != 0 and
+// Above the LDS kernels (n > f64_reg_max_n) the members the gate passes (pf != 0 and
 // the pair pivots' spread within pf_lu_spread_max; psign, the Parlett-Reid run's sign,
 // plog its log|pf|, spread its pivot spread) take pf(S) S^-1 from the blocked LU solves,
 // and the others run the pivot-replaced Parlett-Reid factor and Gauss-Jordan above.

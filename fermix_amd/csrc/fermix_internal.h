@@ -208,7 +208,7 @@ int launch_lu64_small(const double* a, int n, int64_t batch, double* sign, doubl
 // the batch, so not above 1024. Not above n = 512, where panels span several cooperatively
 // launched workgroups that must all be resident.
 inline bool pf_parts_overlap(int64_t batch, int n) { return n <= 512 && batch <= 1024; }
-// float64 blocked LU (sign, logabs) for the orders above the register kernels (lu64_impl.inc)
+// float64 blocked LU (sign, logabs) for the orders above the LDS kernels (lu64_impl.inc)
 size_t lu64_workspace(int64_t batch, int n);
 int launch_lu64(const double* A, int n, int64_t batch, double* sign, double* logabs, void* ws, size_t ws_bytes,
                 hipStream_t s);
@@ -220,7 +220,7 @@ size_t lu64_inverse_workspace(int64_t batch, int n);
 int launch_lu64_inverse(const double* A, int n, int skew, int64_t batch, double* sign, double* logabs,
                         const double* gate, const double* ssign, const double* slog, double* out, int out_t,
                         void* ws, size_t ws_bytes, hipStream_t s, SideStream* side = nullptr);
-// float64 Parlett-Reid sign / logabs for n above the register kernels (lu64_impl.inc): 16 pair
+// float64 Parlett-Reid sign / logabs for n above the LDS kernels (lu64_impl.inc): 16 pair
 // steps per panel, the trailing update on the fp64 MFMA
 size_t pr64_workspace(int64_t batch, int n);
 int launch_pr64_blocked(const double* A, int n, int skew, int64_t batch, double* sign, double* logabs, void* ws,

@@ -269,7 +269,8 @@ __global__ __launch_bounds__(256) void pf_zero_bad_kernel(const int* __restrict_
 }
 
 size_t pf_inverse_workspace(int64_t batch, int N) {
-  if (N <= SMALL_INV_MAXN) return ((size_t)batch * 32 + 255) / 256 * 256;  // nominal, left unused
+  // small_inverse.hip leaves it unused; the entry points ask for a workspace at every order
+  if (N <= SMALL_INV_MAXN) return ((size_t)batch * 32 + 255) / 256 * 256;
   const int Ninv = inv_padded(N);
   size_t bytes = 0;
   auto add = [&](size_t x) { bytes += (x + 255) / 256 * 256; };

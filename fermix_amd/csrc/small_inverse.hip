@@ -185,7 +185,7 @@ __device__ __forceinline__ void solve_lower(const float* T, const int (&j)[2], b
 // d_K the product of the nonzero pivots.
 // Measured, forward + gradient in one process against the embed, diagonal-block inverse, product
 // and guard launches (det: also the parity and pivot launches) that did this before: slogdet
-// B = 4096, n = 100 940 -> 447 us, det B = 16384, n = 24 619 -> 109 us.
+// B = 4096, n = 100 940 -> 392 us, det B = 16384, n = 24 619 -> 102 us.
 template <int NB, bool DET>
 __global__ __launch_bounds__(SmallInv<NB>::NT, SmallInv<NB>::WPE) void lu_inv_small_kernel(
     const float* __restrict__ LU, const int* __restrict__ g0, int n, int64_t batch, const float* __restrict__ sign,
@@ -410,7 +410,7 @@ __device__ __forceinline__ float wedge(float wx, float vy, float vx, float wy) {
 // rows) and are exchanged once through LDS as left operands, 16 bytes per lane; R's lower
 // tiles go back to LDS mirrored and in the output's order. Measured, slogpf forward + gradient
 // B = 2000, n = 90: 520 us as six launches (assembly, inverse, product, vectors, gather,
-// guard) -> 171 us.
+// guard) -> 134 us.
 template <int NB>
 __global__ __launch_bounds__(SmallInv<NB>::NT, SmallInv<NB>::WPE) void pf_inv_small_kernel(
     const float* __restrict__ gbuf, int PB, const float* __restrict__ d, const int* __restrict__ perm, int n,

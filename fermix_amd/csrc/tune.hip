@@ -25,8 +25,8 @@
 //    n = 512 6.32 -> 5.78 ms, n = 1024 9.74 -> 8.64, n = 2048 19.68 -> 17.64, n = 256
 //    4.56 -> 4.41; slogpf fwd + grad 1-4 %;
 //  - f64_reg_max_n 128: float64 in the one-launch kernels (the matrix in LDS) for n <= 128,
-//    the most that 160 KiB hold: B = 1024, n = 128 slogdet 373 us, + A^-T 505, slogpf 230,
-//    + S^-1 775 against 829 / 1800 / 601 / 2490 for the register kernels they replaced and
+//    the most that 160 KiB hold: B = 1024, n = 128 slogdet 396 us, + A^-T 527, slogpf 229,
+//    + S^-1 794 against 829 / 1800 / 601 / 2490 for the register kernels they replaced and
 //    about the same for the blocked ones. f64_strip16_max_n: those kernels' strip width,
 //    without effect since;
 //  - pf_overlap_max_half 32 / pf_overlap_min_work 256: the Parlett-Reid halves with one

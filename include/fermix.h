@@ -26,11 +26,12 @@
  *  - the return value is a status code (FX_OK on success); numerical edge cases are
  *    encoded in the values (an exactly zero pivot gives sign 0 and logabs -inf);
  *  - calls are reentrant; the library keeps no mutable global state apart from the
- *    once-per-device address of the scratch array of fx_slogdet_f32_noalloc, the
- *    once-per-device second stream (and its two events) on which the blocked LU runs
- *    half of a large batch (ordered after the caller's stream and joined back to it
- *    before the call returns; held under a per-device lock while in use) and the
- *    tuning-table override of fx_tune_override;
+ *    once-per-device address of the scratch array of fx_slogdet_f32_noalloc, up to four
+ *    side streams a device (with two events each), on which a call runs an independent part
+ *    of its work (half of a large batch, one triangular factor's inverse, the Parlett-Reid
+ *    beside the LU; ordered after the caller's stream and joined back to it before the
+ *    call returns; one call at a time holds a side stream and no call waits for one) and
+ *    the tuning-table override of fx_tune_override;
  *  - the kernel family is chosen from n alone (never from the batch): several matrices
  *    per wave (n <= 32 for slogdet, 16 for slogpf), one fused workgroup per matrix
  *    (n <= fx_tune.fused_max_n, 128 in the gfx950 table), blocked kernels with workspace
@@ -439,17 +440,16 @@ int fx_slogpf_parts_c128(const double* a, int64_t batch, int32_t n, int32_t skew
                          fx_stream_t stream);
 
 /* adj_t (batch, n, n) = adj(A)^T = d det(A) / dA (holomorphic for complex A, no
- * conjugation) plus sign / logabs of the same Gauss-Jordan run, for float64, complex64
- * and complex128 -- fx_det_parts_f32's contract: det(A) A^-T from the run's own pivots
+ * conjugation) plus the forward's sign / logabs, for float64, complex64 and complex128 -- fx_det_parts_f32's contract: det(A) A^-T from the run's own pivots
  * when no pivot is exactly zero; with zero pivots at columns k1 <= ... <= km (U~ = U with
  * them taken as 1, d_K = the product of the other pivots) the rank-1 continuation
  * sgn(P) d_K c (U~^-1 e_k1)(e_km^T U~^-1 L^-1 P) with c = (U~^-1)[k1, km] for m = 2 and 1
  * for m = 1; 0 for m >= 3 and for a non-finite result. Replaces `_det_gradT` with `_lu_det`
- * and `_perm_sign` (src/fermix/_diff.py:160-246) for the 64-bit and complex kinds. One
- * workgroup per matrix up to n = 128 (float64) / 64 (complex; no workspace while [A | I]
- * fits in 60 KiB of LDS); above, the blocked LU, whose solves give the regular members'
- * det(A) A^-T, the Gauss-Jordan continuation then running only for the exactly singular
- * members. The sign / logabs equal those of fx_slogdet_f64 / _c64 / _c128 (the same
+ * and `_perm_sign` (src/fermix/_diff.py:160-246) for the 64-bit and complex kinds. The
+ * regular members' det(A) A^-T comes from the LU with its inverse (the matrix in LDS up to
+ * n = 128, complex128: 96; the blocked LU and its solves above), the continuation from a
+ * Gauss-Jordan run of the exactly singular members alone, one workgroup per matrix (no
+ * workspace while [A | I] fits in 60 KiB of LDS). The sign / logabs equal those of fx_slogdet_f64 / _c64 / _c128 (the same
  * pivots and per-element updates). */
 size_t fx_det_parts_f64_workspace(int64_t batch, int32_t n);
 int fx_det_parts_f64(const double* a, int64_t batch, int32_t n, double* sign, double* logabs, double* adj_t,

@@ -162,9 +162,9 @@ def test_fused_max_override(dev, n):
 
 @pytest.mark.parametrize("n", [40, 100])
 def test_f64_override(dev, n):
-    """float64 through the LDS / workspace kernel (f64_reg_max_n lowered) and with
-    32-column register strips (f64_strip16_max_n = 0): values and A^-T against numpy's
-    float64, S^-1 against numpy's float64 inverse."""
+    """float64 through the blocked kernels (f64_reg_max_n lowered), and f64_strip16_max_n
+    accepted without effect: values and A^-T against numpy's float64, S^-1 against numpy's
+    float64 inverse."""
     rng = np.random.default_rng(7600 + n)
     A = rng.standard_normal((4, n, n)) / np.sqrt(n)
     S = A - A.transpose(0, 2, 1)
